@@ -63,7 +63,9 @@ typedef struct {
                          0: evaluate every candidate */
   int32_t itile_w;    /* intra fixpoint passes: 8, 16, 32 or 64: a wave settles the reuse
                          chains inside a tile of itile_w x 64/itile_w blocks per pass;
-                         0: exhaustive search re-folds flagged blocks once per pass, learned
+                         0: exhaustive search re-folds flagged blocks once per pass or, where
+                         reuse chains are long (a batch with an intra frame, thresholds from
+                         5 on), decides every block once in dependency order; learned
                          search uses 8 x 8 tiles (same output for every value) */
 } mptc_tuning;
 
@@ -90,7 +92,8 @@ typedef struct {
   int64_t inter_candidates; /* in-frame inter window positions searched */
   int64_t intra_candidates; /* in-frame intra window positions of searched blocks */
   int64_t reeval_candidates;/* intra positions re-evaluated after a word changed */
-  int32_t intra_iterations; /* passes until the intra words reached their fixpoint */
+  int32_t intra_iterations; /* passes until the intra words reached their fixpoint
+                               (1 where every block was decided once) */
   int32_t is_intra;
   int64_t exact_inter_candidates; /* with pruning: candidates evaluated exactly (the rest */
   int64_t exact_intra_candidates; /* were ruled out by the error bound); 0 without pruning */
@@ -173,7 +176,8 @@ int32_t mptc_get_stats(mptc_ctx* ctx, mptc_frame_stats* out);
  * first kernel: counters cleared, fit, reference tables, network input),
  * "inter", "intra_prep" (with the inter decisions of an exhaustive inter
  * search), "intra_dense", "intra_combine",
- * "intra_apply", "intra_reeval", "intra_tile", "commit", "unique";
+ * "intra_apply", "intra_reeval", "intra_tile", "intra_wave" (the decisions in
+ * dependency order), "commit", "unique";
  * learned search: "net_input", "net_l12", "net_l3" (inference), "propose_inter",
  * "top_intra", "lintra_pass"; "net_forward": training steps (the fused
  * forward/loss/backward, weight-gradient and reduction/Adam launches); pruned search:

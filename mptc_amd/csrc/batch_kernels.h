@@ -81,6 +81,7 @@ struct DevStats {
   unsigned int n_changed[2];             // length of the changed-word list, by pass parity
   unsigned int pass_done;                // workgroups of the running fixpoint pass that finished
   unsigned int skip_tile;                // the last pass was tile-resolved (k_intra_tile_pass)
+  unsigned int wave_ticket, wave_done, wave_fail;  // k_intra_wave: rows taken, rows finished, a row gave up
   unsigned int pass_grp[kPassGroups * kPassStride];  // pass_end's group counters
 };
 
@@ -404,13 +405,16 @@ __device__ __forceinline__ uint64_t inter_decision(const FrameDev& d, int g, int
 // the chunk summaries and write them to inter_dec; otherwise inter_dec holds
 // them already (learned proposals).  With orig_ready the blocks of inter
 // frames already have their own error in orig (the pruned inter search).
+// fin (null: not wanted) receives the words k_intra_wave starts from, rec its
+// block records (it may be summ: a block's record replaces its own first
+// chunk summary, which only its thread reads).
 __global__ void __launch_bounds__(256) k_intra_prep(const FrameDev* __restrict__ fr, const uint8_t* __restrict__ sid, int total,
                              const uint64_t* __restrict__ own, uint64_t* __restrict__ inter_dec,
                              uint8_t* __restrict__ need, uint32_t* __restrict__ cw, float4* __restrict__ ctab,
                              uint32_t* __restrict__ dirty, int* __restrict__ orig, BoundTab* __restrict__ cbt,
                              uint4* __restrict__ pm4, int n_chunks, int S, int thr,
-                             const uint32_t* __restrict__ rw, const uint4* __restrict__ summ, size_t sstride,
-                             int orig_ready) {
+                             const uint32_t* __restrict__ rw, const uint4* summ, size_t sstride,
+                             int orig_ready, uint64_t* __restrict__ fin, uint4* rec) {
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= total) return;
   const FrameDev& d = fr[sid[g]];
@@ -433,6 +437,7 @@ __global__ void __launch_bounds__(256) k_intra_prep(const FrameDev* __restrict__
   }
   need[g] = inter_ok ? 0 : 1;
   cw[g] = w;
+  if (fin) fin[g] = (inter_ok ? 1ull << 63 : 0ull) | (uint64_t)g << 32 | w;
   if (!orig) return;  // the learned intra search builds its own tables and errors
   dirty[g] = 0;
   const CandTab t = cand_table(w);
@@ -442,10 +447,17 @@ __global__ void __launch_bounds__(256) k_intra_prep(const FrameDev* __restrict__
     pm4[2 * g] = make_uint4(0u, 0u, 0u, 0u);
     pm4[2 * g + 1] = make_uint4(0u, 0u, 0u, 0u);
   }
-  if (orig_ready && !d.is_intra) return;  // the pruned inter search wrote the own error
-  BlockPx px;
-  load_block(d.rgb, d.width, k % d.bw, k / d.bw, px);
-  orig[g] = own_error(px, o);
+  int err;
+  if (orig_ready && !d.is_intra) {  // the pruned inter search wrote the own error
+    if (!fin) return;
+    err = orig[g];
+  } else {
+    BlockPx px;
+    load_block(d.rgb, d.width, k % d.bw, k / d.bw, px);
+    err = own_error(px, o);
+    orig[g] = err;
+  }
+  if (fin) rec[g] = make_uint4((uint32_t)(o >> 32), (uint32_t)err, inter_ok ? 0u : 1u, 0u);
 }
 
 // Intra scan order (codec/dxt_image.cpp:672-675): rows j = by .. by-2S+1

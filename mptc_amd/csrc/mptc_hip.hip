@@ -26,6 +26,7 @@
 #include "../../include/mptc.h"
 #include "net_infer.h"
 #include "prune_kernels.h"
+#include "wave_kernels.h"
 #include "framegen.h"
 
 using namespace mptc;
@@ -99,6 +100,9 @@ int init_tables(int device) {
   HIP_TRY(hipMemcpyToSymbol(HIP_SYMBOL(c_omatch5), om5, sizeof(om5)));
   HIP_TRY(hipMemcpyToSymbol(HIP_SYMBOL(c_omatch6), om6, sizeof(om6)));
   HIP_TRY(hipMemcpyToSymbol(HIP_SYMBOL(c_snap), snap, sizeof(snap)));
+  for (auto kern : {k_intra_wave<0>, k_intra_wave<8>, k_intra_wave<16>, k_intra_wave<32>})
+    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                wave_dims(kWaveMaxS).bytes));
   done[device] = true;
   return MPTC_OK;
 }
@@ -106,35 +110,35 @@ int init_tables(int device) {
 enum KernelId {
   KF_FIT, KF_INTER, KF_PREP, KF_DENSE, KF_INTRA_COMBINE, KF_APPLY, KF_REEVAL,
   KF_TILE, KF_COMMIT, KF_UNIQUE, KF_NET_INPUT, KF_NET_FWD, KF_PROPOSE, KF_TOP_INTRA, KF_LPASS, KF_NET_L12,
-  KF_NET_L3, KF_PRUNED_INTER, KF_PRUNED_INTRA, KF_FOLD_INTRA, KF_N
+  KF_NET_L3, KF_PRUNED_INTER, KF_PRUNED_INTRA, KF_FOLD_INTRA, KF_WAVE, KF_N
 };
 const char* kKernelNames[KF_N] = {"fit",          "inter",
                                   "intra_prep",   "intra_dense", "intra_combine",
                                   "intra_apply",  "intra_reeval", "intra_tile", "commit",
                                   "unique",       "net_input",   "net_forward", "propose_inter",
                                   "top_intra",    "lintra_pass",  "net_l12",     "net_l3",
-                                  "pruned_inter", "pruned_intra", "fold_intra"};
+                                  "pruned_inter", "pruned_intra", "fold_intra",  "intra_wave"};
 constexpr int kMaxChunks = 8;  // window-row chunks per block in the search kernels
 
 constexpr int kReevalGrid = 1024;  // workgroups of the re-evaluation pass (grid-stride; 1024 measured faster than 4096)
 constexpr int kListGrid = 256;     // workgroups of the list-apply pass (grid-stride)
 
 struct Graphs {
-  hipGraphExec_t prefix = nullptr, passes = nullptr, suffix = nullptr;
+  hipGraphExec_t prefix = nullptr, passes = nullptr, wave = nullptr, suffix = nullptr;
   void destroy() {
     if (prefix) (void)hipGraphExecDestroy(prefix);
     if (passes) (void)hipGraphExecDestroy(passes);
+    if (wave) (void)hipGraphExecDestroy(wave);
     if (suffix) (void)hipGraphExecDestroy(suffix);
-    prefix = passes = suffix = nullptr;
+    prefix = passes = wave = suffix = nullptr;
   }
 };
-// The step's graphs for a batch with inter frames (v[1]) and for a batch of
-// intra frames only (v[0]), which skips the inter search.
+// The step's graphs for a batch of intra frames only (v[0]: no inter search),
+// of inter frames only (v[1]) and of both (v[2]).
 struct GraphSet {
-  Graphs v[2];
+  Graphs v[3];
   void destroy() {
-    v[0].destroy();
-    v[1].destroy();
+    for (Graphs& g : v) g.destroy();
   }
 };
 
@@ -197,6 +201,9 @@ struct mptc_ctx {
   uint32_t *d_rw = nullptr, *d_cw = nullptr, *d_cwn = nullptr, *d_dirty = nullptr, *d_tiles = nullptr;
   float4 *d_rtab = nullptr, *d_ctab = nullptr;
   int *d_orig = nullptr, *d_chg = nullptr;
+  uint64_t* d_fin = nullptr;  // k_intra_wave: words, final from bit 32
+  int* d_wrows = nullptr;     // its rows in ticket order (null: one frame, rows in order)
+  int n_wrows = 0;
   uint2* d_E = nullptr;  // S^2 groups of four int16 error deltas per block
   uint4* d_summ = nullptr;  // kMaxChunks selection summaries per block
   DevStats* d_stats = nullptr;
@@ -214,7 +221,8 @@ struct mptc_ctx {
   mptc_tuning shape_tune{0, 0, 0, 0, 0, 0, 0};
   int n_frames = 0, total = 0, n_wtiles = 0, n_tiles = 0, n_itiles = 0;
   GraphSet graphs;
-  bool any_inter = true;  // the batch holds an inter frame
+  bool any_inter = true;   // the batch holds an inter frame
+  bool any_intra = false;  // and an intra frame
   int last_passes = 0, last_total = 0, last_intra = 0;
   // learned proposals
   int mode = MPTC_SEARCH_EXHAUSTIVE, top_k = 8;
@@ -482,13 +490,32 @@ int prepare_batch(mptc_ctx* c, hipStream_t s, int n, const FrameIn* in) {
     hipLaunchKernelGGL(k_fill_sid, dim3(grid_for(maxnb, 256), n), dim3(256), 0, s, c->d_fr, n, c->d_sid);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s));  // the tsid staging vector is released on return
+    if (c->d_wrows) (void)hipFree(c->d_wrows);
+    c->d_wrows = nullptr;
+    if (n > 1) {  // k_intra_wave's rows: every frame's first, then every frame's second, ...
+      std::vector<int> rows;
+      int maxh = 0;
+      for (int f = 0; f < n; ++f) maxh = std::max(maxh, h[f].bh);
+      for (int y = 0; y < maxh; ++y)
+        for (int f = 0; f < n; ++f)
+          if (y < h[f].bh) rows.push_back(y << 6 | f);
+      if ((rc = dalloc(&c->d_wrows, rows.size()))) return rc;
+      HIP_TRY(hipMemcpyAsync(c->d_wrows, rows.data(), sizeof(int) * rows.size(), hipMemcpyHostToDevice, s));
+      HIP_TRY(hipStreamSynchronize(s));
+    }
     c->graphs.destroy();
     c->shape = shape;
     c->shape_tune = c->tune;
   }
   c->n_frames = n;
+  c->n_wrows = 0;
+  for (int f = 0; f < n; ++f) c->n_wrows += h[f].bh;
   c->any_inter = false;
-  for (int f = 0; f < n; ++f) c->any_inter = c->any_inter || !in[f].is_intra;
+  c->any_intra = false;
+  for (int f = 0; f < n; ++f) {
+    c->any_inter = c->any_inter || !in[f].is_intra;
+    c->any_intra = c->any_intra || in[f].is_intra;
+  }
   c->total = base;
   c->n_wtiles = wt;
   c->n_tiles = tb;
@@ -570,9 +597,53 @@ int lintra_pass_q(mptc_ctx* c, hipStream_t s, int par, int first, bool report) {
   });
 }
 
+// Whether a step's exhaustive intra decisions are taken in dependency order
+// (k_intra_wave) instead of by fixpoint passes: no recording (its acceptance
+// sets are the fixpoint's deltas), no tile passes asked for, and
+//  - a frame of the batch is intra: reuse chains run through all of it.  An
+//    inter frame's few searching blocks settle in about 8 passes (1080p,
+//    S = 8, threshold 8: 0.84 ms a frame with the passes, 2.8 with the wave);
+//  - the threshold is high enough for words to be reused widely.  1080p intra
+//    frames, S = 8, ms a frame, passes / wave: threshold 2 1.3 / 5.8, 4 5.2 / 5.5,
+//    8 23 / 4.8, 32 40 / 4.3; S = 32: 8 288 / 25, 32 770 / 12;
+//  - above S = 16, where a window may hold more distinct words than there are
+//    ids (1080p, S = 32: up to 2,100 at threshold 4, 800 at 8), from 8 on.
+constexpr int kWaveMinThr = 5, kWaveWideS = 16, kWaveWideThr = 8;
+
+bool use_wave(const mptc_ctx* c) {
+  const int S = c->cfg.search_area;
+  return c->mode != MPTC_SEARCH_LEARNED && !c->record && c->tune.itile_w == 0 && c->any_intra && S <= kWaveMaxS &&
+         c->cfg.err_threshold >= (S <= kWaveWideS ? kWaveMinThr : kWaveWideThr);
+}
+
+int queue_wave(mptc_ctx* c, hipStream_t s) {
+  const int S = c->cfg.search_area;
+  return launch(c, s, KF_WAVE, [&] {
+    auto kern = S == 8 ? k_intra_wave<8> : S == 16 ? k_intra_wave<16> : S == 32 ? k_intra_wave<32> : k_intra_wave<0>;
+    hipLaunchKernelGGL(kern, dim3(c->n_wrows), dim3(64 * kWaveWaves), wave_dims(S).bytes, s, c->d_fr,
+                       c->n_frames > 1 ? c->d_wrows : nullptr, S, c->cfg.err_threshold, c->d_summ, c->d_ctab,
+                       c->d_fin, c->d_intra, c->d_stats, c->d_conv);
+  });
+}
+
+// k_intra_prep: the intra search's start, from the inter decisions (taken from
+// inter_summ's chunk summaries where it is given); wave: k_intra_wave's too.
+int queue_intra_prep(mptc_ctx* c, hipStream_t s, bool prune, bool wave, const uint4* inter_summ, int orig_ready) {
+  const int total = c->total, wg = c->tune.wg_size, S = c->cfg.search_area;
+  const bool lrn = c->mode == MPTC_SEARCH_LEARNED;  // its intra passes use no tables, errors or flags
+  return launch(c, s, KF_PREP, [&] {
+    hipLaunchKernelGGL(k_intra_prep, dim3(grid_for(total, wg)), dim3(wg), 0, s, c->d_fr, c->d_sid, total, c->d_own,
+                       c->d_inter, c->d_need, c->d_cw, lrn ? nullptr : c->d_ctab, lrn ? nullptr : c->d_dirty,
+                       lrn ? nullptr : c->d_orig, prune ? c->d_cbt : nullptr,
+                       prune ? reinterpret_cast<uint4*>(c->d_pm) : nullptr, chunks_for(S, c->tune.win_chunks), S,
+                       c->cfg.err_threshold, c->d_rw, inter_summ, c->nbs, orig_ready, wave ? c->d_fin : nullptr, c->d_summ);
+  });
+}
+
 // The three launch sequences of a step.  `fit` = false starts from
-// caller-provided fitted blocks already in d_own.
-int queue_prefix(mptc_ctx* c, hipStream_t s, bool fit) {
+// caller-provided fitted blocks already in d_own; `wave`: k_intra_wave follows
+// (no intra candidates evaluated here).
+int queue_prefix(mptc_ctx* c, hipStream_t s, bool fit, bool wave) {
   const int total = c->total, wg = c->tune.wg_size, tw = c->tune.tile_w;
   const int S = c->cfg.search_area, thr = c->cfg.err_threshold;
   int rc;
@@ -582,7 +653,7 @@ int queue_prefix(mptc_ctx* c, hipStream_t s, bool fit) {
                        (c->mode == MPTC_SEARCH_LEARNED && !c->net[MPTC_NET_INTRA].use_prior));
   bool x_done = want_x;
   bool prep_done = false;  // need and the starting intra words already set
-  const bool prune = use_prune(c);
+  const bool prune = use_prune(c) && !wave;
   if ((rc = launch(c, s, KF_FIT, [&] {
          const int n_st = (int)(sizeof(DevStats) / 4);
          hipLaunchKernelGGL(k_block_prep, dim3(grid_for(std::max(total, n_st + c->n_tiles), wg)), dim3(wg), 0, s,
@@ -631,15 +702,8 @@ int queue_prefix(mptc_ctx* c, hipStream_t s, bool fit) {
          })))
       return rc;
   }
-  if (!prep_done && (rc = launch(c, s, KF_PREP, [&] {
-         const bool lrn = c->mode == MPTC_SEARCH_LEARNED;  // its intra passes use no tables, errors or flags
-         hipLaunchKernelGGL(k_intra_prep, dim3(grid_for(total, wg)), dim3(wg), 0, s, c->d_fr, c->d_sid, total,
-                            c->d_own, c->d_inter, c->d_need, c->d_cw, lrn ? nullptr : c->d_ctab,
-                            lrn ? nullptr : c->d_dirty, lrn ? nullptr : c->d_orig, prune ? c->d_cbt : nullptr,
-                            prune ? reinterpret_cast<uint4*>(c->d_pm) : nullptr, K, S, thr, c->d_rw, inter_summ,
-                            c->nbs, orig_ready);
-       })))
-    return rc;
+  if (!prep_done && (rc = queue_intra_prep(c, s, prune, wave, inter_summ, orig_ready))) return rc;
+  if (wave) return MPTC_OK;
   if (c->mode == MPTC_SEARCH_LEARNED) {
     if ((rc = proposals_q(c, s, MPTC_NET_INTRA, c->d_need, c->d_prop, x_done))) return rc;
     return lintra_pass_q(c, s, 0, 1, false);
@@ -765,27 +829,54 @@ int capture(hipStream_t s, hipGraphExec_t* exec, Q&& q) {
 // One encode step over the prepared batch.
 int run_step(mptc_ctx* c, hipStream_t s, bool fit) {
   const bool graphs = c->tune.use_graph && !c->prof && fit;
-  Graphs& gr = c->graphs.v[c->any_inter ? 1 : 0];
+  Graphs& gr = c->graphs.v[!c->any_inter ? 0 : c->any_intra ? 2 : 1];
   int rc;
   // The last pass of each batch writes its count of changed words to h_conv
   // (0 when it had nothing to do).  Passes of an earlier step that are still
   // queued can only write 0 (they follow a pass that changed nothing), and
   // they run before this step's passes on the ordered stream.
-  *reinterpret_cast<volatile uint32_t*>(c->h_conv) = 0u;
+  volatile uint32_t* conv = c->h_conv;
+  *conv = 0u;
+  const bool wave = use_wave(c);
   if (graphs && !gr.prefix) {
-    if ((rc = capture(s, &gr.prefix, [&] { return queue_prefix(c, s, true); }))) return rc;
+    if ((rc = capture(s, &gr.prefix, [&] { return queue_prefix(c, s, true, wave); }))) return rc;
     if ((rc = capture(s, &gr.passes, [&] { return queue_passes(c, s); }))) return rc;
+    if (wave && (rc = capture(s, &gr.wave, [&] { return queue_wave(c, s); }))) return rc;
     if ((rc = capture(s, &gr.suffix, [&] { return queue_suffix(c, s); }))) return rc;
   }
   if (graphs) {
     HIP_TRY(hipGraphLaunch(gr.prefix, s));
-  } else if ((rc = queue_prefix(c, s, fit))) {
+  } else if ((rc = queue_prefix(c, s, fit, wave))) {
     return rc;
   }
   if (c->batch_ev.empty()) {
     c->batch_ev.resize(2);
     for (auto& e : c->batch_ev) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   }
+  // poll (a blocking wait adds its wake-up latency to every batch)
+  auto wait = [&](int slot) -> int {
+    hipError_t q;
+    while ((q = hipEventQuery(c->batch_ev[slot])) == hipErrorNotReady) {
+    }
+    if (q != hipSuccess) return fail(MPTC_EHIP, std::string("hipEventQuery: ") + hipGetErrorString(q));
+    return MPTC_OK;
+  };
+  // k_intra_wave over the whole batch; false in `ok`: a window held more
+  // distinct words than it has ids for, and the passes start over
+  auto run_wave = [&](bool& ok) -> int {
+    int r;
+    if (graphs) {
+      HIP_TRY(hipGraphLaunch(gr.wave, s));
+    } else if ((r = queue_wave(c, s))) {
+      return r;
+    }
+    HIP_TRY(hipEventRecord(c->batch_ev[0], s));
+    if ((r = wait(0))) return r;
+    ok = *conv == 0;
+    return ok ? MPTC_OK : queue_prefix(c, s, fit, false);
+  };
+  bool settled = false;
+  if (wave && (rc = run_wave(settled))) return rc;
   const int np = passes_per_batch(c);
   int passes = 0;
   auto queue_batch = [&](int slot) -> int {
@@ -800,22 +891,18 @@ int run_step(mptc_ctx* c, hipStream_t s, bool fit) {
     return MPTC_OK;
   };
   int slot = 0;
-  if ((rc = queue_batch(slot))) return rc;
-  for (;;) {
+  if (!settled && (rc = queue_batch(slot))) return rc;
+  while (!settled) {
     // the raster-triangular system settles within one pass per block
     if (passes > c->total + 4 * np) return fail(MPTC_ESTATE, "intra fixpoint did not converge");
     if ((rc = queue_batch(slot ^ 1))) return rc;
-    // poll (a blocking wait adds its wake-up latency to every batch)
-    hipError_t q;
-    while ((q = hipEventQuery(c->batch_ev[slot])) == hipErrorNotReady) {
-    }
-    if (q != hipSuccess) return fail(MPTC_EHIP, std::string("hipEventQuery: ") + hipGetErrorString(q));
+    if ((rc = wait(slot))) return rc;
     // The last pass of every batch writes its count of changed words to
     // h_conv, so once the batch is done h_conv holds the count of its last
     // pass or of a later batch's last pass.  A pass that changes nothing
     // proves the fixpoint (every later pass is empty too); the batch queued
     // after it then runs empty.
-    if (*reinterpret_cast<volatile uint32_t*>(c->h_conv) == 0) break;
+    if (*conv == 0) break;
     slot ^= 1;
   }
   if (graphs) {
@@ -899,7 +986,7 @@ int32_t mptc_create(const mptc_config* cfg, mptc_ctx** out) {
       (rc = dalloc(&c->d_own, nb)) || (rc = dalloc(&c->d_inter, nb)) || (rc = dalloc(&c->d_intra, nb)) ||
       (rc = dalloc(&c->d_rw, nb)) || (rc = dalloc(&c->d_cw, nb)) || (rc = dalloc(&c->d_cwn, nb)) ||
       (rc = dalloc(&c->d_dirty, nb)) || (rc = dalloc(&c->d_tiles, max_tiles)) || (rc = dalloc(&c->d_rtab, nb)) ||
-      (rc = dalloc(&c->d_ctab, nb)) || (rc = dalloc(&c->d_orig, nb)) || (rc = dalloc(&c->d_chg, nb)) ||
+      (rc = dalloc(&c->d_ctab, nb)) || (rc = dalloc(&c->d_orig, nb)) || (rc = dalloc(&c->d_chg, nb)) || (rc = dalloc(&c->d_fin, nb)) ||
       (rc = dalloc(&c->d_E, groups * c->nbs)) || (rc = dalloc(&c->d_summ, kMaxChunks * c->nbs)) || (rc = dalloc(&c->d_stats, 1)) ||
       (rc = dalloc(&c->d_rgb, one_nb * 48)) || (rc = dalloc(&c->d_ref, one_nb)) || (rc = dalloc(&c->d_phys, one_nb)) ||
       (rc = dalloc(&c->d_motion, one_nb * 2)) || (rc = dalloc(&c->d_eps, one_nb * 6)) ||
@@ -930,7 +1017,7 @@ void mptc_destroy(mptc_ctx* c) {
   for (hipEvent_t e : c->batch_ev) (void)hipEventDestroy(e);
   void* bufs[] = {c->d_fr,   c->d_sid,   c->d_tsid,   c->d_need,  c->d_own,   c->d_inter,  c->d_intra,
                   c->d_rw,   c->d_cw,    c->d_cwn,    c->d_dirty, c->d_tiles, c->d_rtab,   c->d_ctab,
-                  c->d_orig, c->d_chg,   c->d_E, c->d_summ,     c->d_stats, c->d_rgb,    c->d_ref,
+                  c->d_orig, c->d_chg,   c->d_fin,    c->d_wrows, c->d_E, c->d_summ,     c->d_stats, c->d_rgb,    c->d_ref,
                   c->d_phys, c->d_motion, c->d_eps,   c->d_kind,  c->d_unique, c->d_nunique};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
@@ -1551,7 +1638,7 @@ constexpr size_t kNaNbs = kNaMaxBlocks;  // E row stride, a multiple of 64
 
 enum NaBuf {
   NA_FR, NA_SID, NA_TSID, NA_NEED, NA_OWN, NA_INTER, NA_INTRA, NA_RW, NA_CW, NA_CWN, NA_DIRTY, NA_TILES,
-  NA_RTAB, NA_CTAB, NA_ORIG, NA_CHG, NA_E, NA_SUMM, NA_STATS, NA_RBT, NA_CBT, NA_PM, NA_CONV, NA_N
+  NA_RTAB, NA_CTAB, NA_ORIG, NA_CHG, NA_FIN, NA_E, NA_SUMM, NA_STATS, NA_RBT, NA_CBT, NA_PM, NA_CONV, NA_N
 };
 
 constexpr size_t na_align(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
@@ -1562,7 +1649,7 @@ constexpr size_t na_bytes(int b) {
   switch (b) {
     case NA_FR: return sizeof(FrameDev);
     case NA_SID: case NA_TSID: case NA_NEED: return kNaNbs;  // a wave tile holds at least one block
-    case NA_OWN: case NA_INTER: case NA_INTRA: return 8 * kNaNbs;
+    case NA_OWN: case NA_INTER: case NA_INTRA: case NA_FIN: return 8 * kNaNbs;
     case NA_RW: case NA_CW: case NA_CWN: case NA_DIRTY: case NA_ORIG: case NA_CHG: return 4 * kNaNbs;
     case NA_TILES: return 4 * (kNaMaxBlocks / kUniqueTile + 2);
     case NA_RTAB: case NA_CTAB: return sizeof(float4) * kNaNbs;
@@ -1639,6 +1726,7 @@ int na_setup(int device, NoAllocDev& nd) {
   c.d_ctab = static_cast<float4*>(at(NA_CTAB));
   c.d_orig = static_cast<int*>(at(NA_ORIG));
   c.d_chg = static_cast<int*>(at(NA_CHG));
+  c.d_fin = static_cast<uint64_t*>(at(NA_FIN));
   c.d_E = static_cast<uint2*>(at(NA_E));
   c.d_summ = static_cast<uint4*>(at(NA_SUMM));
   c.d_stats = static_cast<DevStats*>(at(NA_STATS));
@@ -1705,17 +1793,33 @@ int32_t mptc_encode_frame_noalloc(int32_t device, const uint8_t* d_rgb, int32_t 
   c->n_tiles = tb;
   c->n_itiles = lt;
   c->any_inter = !is_intra;
+  c->any_intra = is_intra;
   c->last_intra = is_intra;
-  if ((rc = queue_prefix(c, s, true))) return rc;
-  // fixpoint passes in batches; after each batch the count of changed words
-  // of its last pass comes back by a plain copy (no event, no mapped memory)
-  const int np = passes_per_batch(c);
-  for (int passes = 0;; passes += np) {
-    if (passes > c->total + 4 * np) return fail(MPTC_ESTATE, "intra fixpoint did not converge");
-    if ((rc = queue_passes(c, s))) return rc;
+  c->n_wrows = nd.h_fr.bh;
+  // the status word of the passes or the wave comes back by a plain copy (no
+  // event, no mapped memory)
+  auto status = [&]() -> int {
     HIP_TRY(hipMemcpyAsync(&nd.h_changed, c->d_conv, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    if (nd.h_changed == 0) break;
+    return MPTC_OK;
+  };
+  bool settled = false, wave = use_wave(c);
+  if ((rc = queue_prefix(c, s, true, wave))) return rc;
+  // fixpoint passes in batches; after each batch the count of changed words
+  // of its last pass
+  const int np = passes_per_batch(c);
+  for (int passes = 0; !settled;) {
+    if (wave) {
+      wave = false;
+      if ((rc = queue_wave(c, s)) || (rc = status())) return rc;
+      settled = nd.h_changed == 0;
+      if (!settled && (rc = queue_prefix(c, s, true, false))) return rc;
+      continue;
+    }
+    if (passes > c->total + 4 * np) return fail(MPTC_ESTATE, "intra fixpoint did not converge");
+    if ((rc = queue_passes(c, s)) || (rc = status())) return rc;
+    passes += np;
+    settled = nd.h_changed == 0;
   }
   if ((rc = queue_suffix(c, s))) return rc;
   HIP_TRY(hipStreamSynchronize(s));  // the frame is done when the call returns

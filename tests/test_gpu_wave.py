@@ -1,0 +1,96 @@
+"""Intra search in dependency order (k_intra_wave) against the CPU oracle, at
+the sizes where its window, its rings and its id tables have their edges."""
+from __future__ import annotations
+
+import sys
+
+import numpy as np
+import pytest
+
+from tests.helpers import compare_results
+
+pytestmark = pytest.mark.gpu
+
+
+def log(msg: str):
+    print(msg, flush=True)
+    sys.stdout.flush()
+
+
+@pytest.fixture(scope="module")
+def enc():
+    from mptc_amd import lib
+    e = lib.Encoder(512, 512, search_area=32, err_threshold=0, max_batch_frames=3, max_batch_blocks=3 * 128 * 128)
+    yield e
+    e.close()
+
+
+def _frame(kind: str, w: int, h: int, seed: int) -> np.ndarray:
+    rng = np.random.default_rng(seed)
+    if kind == "noise":  # words that few blocks can reuse
+        return rng.integers(0, 256, (h, w, 3)).astype(np.uint8)
+    yy, xx = np.mgrid[0:h, 0:w]
+    img = np.stack([30 + xx // 3, 60 + yy // 2, 200 - (xx + yy) // 5], -1)
+    if kind == "flat":  # wide steps: equal words, blocks that keep their own
+        return np.clip(img // 32 * 32, 0, 255).astype(np.uint8)
+    return np.clip(img + rng.integers(-8, 9, (h, w, 3)), 0, 255).astype(np.uint8)
+
+
+def _intra(enc, orc, rgb, S, thr):
+    enc.set_params(S, thr)
+    fit = enc.fit(rgb)
+    got = enc.reencode(rgb, fit, True)
+    want = orc.reencode(rgb, fit, S, thr, True)
+    compare_results(got, want, f"{rgb.shape[1]}x{rgb.shape[0]} S={S} thr={thr}")
+    assert np.array_equal(got["kind"], want["kind"])
+
+
+# one block; one row; one column; narrower and wider than the window; rows of 15, 16, 17 and 63-65 blocks (staging
+# groups, polled vectors, need chunks); S at its ends, odd, and past the ring and id sizes' steps
+@pytest.mark.parametrize("kind,w,h,S,thr", [
+    ("soft", 4, 4, 1, 8), ("soft", 260, 4, 8, 8), ("soft", 4, 200, 8, 8), ("soft", 28, 60, 8, 5), ("soft", 60, 40, 8, 8),
+    ("soft", 64, 48, 1, 8), ("soft", 68, 48, 2, 30), ("flat", 68, 52, 3, 8), ("soft", 252, 64, 4, 8), ("soft", 256, 64, 5, 16),
+    ("soft", 260, 64, 7, 8), ("soft", 300, 120, 8, 30000), ("flat", 300, 120, 8, 8), ("noise", 200, 100, 8, 300),
+    ("soft", 200, 100, 9, 8), ("soft", 220, 96, 15, 8), ("soft", 220, 96, 16, 6), ("noise", 160, 160, 16, 900),
+    ("soft", 260, 132, 17, 8), ("soft", 300, 140, 31, 12), ("soft", 300, 140, 32, 8), ("flat", 264, 132, 32, 32)])
+def test_intra_wave_matches_oracle(enc, orc, kind, w, h, S, thr):
+    log(f"{kind} {w}x{h} S={S} thr={thr}")
+    enc.profile_enable(True)
+    _intra(enc, orc, _frame(kind, w, h, w + h + S), S, thr)
+    launches, _ = enc.profile_read("intra_wave")
+    enc.profile_enable(False)
+    assert launches == 1
+
+
+def test_more_distinct_words_than_ids(enc, orc):
+    """A noise frame holds more distinct words than the S = 32 window has ids:
+    the fixpoint passes take over, with the same result."""
+    rgb = _frame("noise", 300, 280, 5)
+    enc.profile_enable(True)
+    _intra(enc, orc, rgb, 32, 8)
+    waves, passes = enc.profile_read("intra_wave")[0], enc.profile_read("intra_reeval")[0]
+    enc.profile_enable(False)
+    assert waves == 1 and passes > 0
+
+
+def test_batch_of_intra_and_inter_frames(enc, orc):
+    """One call with intra and inter frames of uneven sizes: every frame as by itself."""
+    from mptc_amd import hip
+    S, thr = 8, 8
+    enc.set_params(S, thr)
+    jobs, want = [], []
+    for i, (w, h, intra) in enumerate([(200, 100, True), (64, 120, False), (324, 36, True)]):
+        a, b = _frame("soft", w, h, 10 + i), _frame("soft", w, h, 20 + i)
+        nb = (w // 4) * (h // 4)
+        ref = orc.reencode(a, orc.fit_frame(a), S, thr, True)["phys"]
+        want.append(orc.reencode(b, orc.fit_frame(b), S, thr, intra, None if intra else ref))
+        jobs.append(dict(d_rgb=hip.Buffer.from_array(b), width=w, height=h, is_intra=intra, d_ref=hip.Buffer.from_array(ref),
+                         d_phys=hip.Buffer(8 * nb), d_motion=hip.Buffer(2 * nb), d_unique=hip.Buffer(4 * nb),
+                         d_n_unique=hip.Buffer(4), d_eps=hip.Buffer(6 * nb), d_kind=hip.Buffer(nb)))
+    enc.encode_batch_device(jobs)
+    for i, (j, wnt) in enumerate(zip(jobs, want)):
+        nb = (j["width"] // 4) * (j["height"] // 4)
+        n = int(j["d_n_unique"].download(np.uint32, 1)[0])
+        got = dict(phys=j["d_phys"].download(np.uint64, nb), motion=j["d_motion"].download(np.uint8, 2 * nb),
+                   unique=j["d_unique"].download(np.uint32, n), eps=j["d_eps"].download(np.uint8, 6 * nb))
+        compare_results(got, wnt, f"frame {i}")
