@@ -479,10 +479,9 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
           if (kept != id && (kept & 63u) < kAboveIds && (uint32_t)wr[kept] == w) id = kept;
         }
         if (fresh) {
-          if (id == mine) {
-            if (!t_ok) t0 = ctab[fin_root(v)];
-            tab[id] = t0;
-          }
+          // an id given up for an equal word's keeps this word (a bucket may still name it), so its table too
+          if (!t_ok) t0 = ctab[fin_root(v)];
+          tab[mine] = t0;
           atomicMax(&lastany[id], seen);
         }
       }

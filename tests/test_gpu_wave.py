@@ -94,3 +94,22 @@ def test_batch_of_intra_and_inter_frames(enc, orc):
         got = dict(phys=j["d_phys"].download(np.uint64, nb), motion=j["d_motion"].download(np.uint8, 2 * nb),
                    unique=j["d_unique"].download(np.uint32, n), eps=j["d_eps"].download(np.uint8, 6 * nb))
         compare_results(got, wnt, f"frame {i}")
+
+
+@pytest.mark.parametrize("w,h,S,thr,seed", [(1920, 1080, 8, 8, 3), (1280, 720, 16, 8, 4), (960, 540, 32, 16, 5)])
+def test_intra_wave_matches_tile_passes(w, h, S, thr, seed):
+    """Ordinary frame sizes, where ids are given out and taken back thousands of
+    times a row: the same bytes as the tile-resolved fixpoint passes, and the
+    same from one encode to the next."""
+    from mptc_amd import lib
+    from mptc_amd.workloads import SynthCfg
+    rgb = lib.synth_frames(SynthCfg(w, h, seed, 32, 1, 4, 8, 10), 0, 1)[0]
+    e = lib.Encoder(w, h, S, thr)
+    fit = e.fit(rgb)
+    runs = [e.reencode(rgb, fit, True) for _ in range(4)]
+    e.set_tuning(itile_w=8)
+    want = e.reencode(rgb, fit, True)
+    e.close()
+    for i, r in enumerate(runs):
+        compare_results(r, want, f"{w}x{h} S={S} thr={thr} run {i}")
+        assert np.array_equal(r["kind"], want["kind"])
