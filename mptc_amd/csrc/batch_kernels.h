@@ -65,11 +65,13 @@ constexpr int kStatSlots = 32;
 constexpr int kSlot64 = 16;
 constexpr int kSlot32 = 32;
 
-// pass_end counts finished workgroups in two levels: groups of kPassGroup
-// workgroups count into their own counter (one 256-byte line each), and the
-// last workgroup of each group into pass_done.
+// pass_end counts finished workgroups in two levels: at most kPassGroups groups
+// of at least kPassGroup workgroups count into their own counter (one 256-byte
+// line each), and the last workgroup of each group into pass_done.  Larger
+// grids have larger groups: 8,438 workgroups (2.16 M blocks) on one counter
+// queued for 100 us a pass, in 64 groups of 132 the pass takes 22.
 constexpr int kPassGroup = 64;
-constexpr int kPassGroups = 64;  // grids of up to 4,096 workgroups; larger ones count flat
+constexpr int kPassGroups = 64;
 constexpr int kPassStride = 64;  // words between the group counters
 
 struct DevStats {
@@ -148,15 +150,17 @@ __device__ __forceinline__ void wg_count(unsigned long long* s_acc, unsigned lon
 // The workgroups' counter updates are atomics whose results they consume
 // before they get here, so they are complete before their count (no
 // device-scope fence, which would write back the XCD's L2).  The count is
-// two-level (kPassGroup workgroups per group counter, then the groups), so
+// two-level (the workgroups of a group, then the groups), so
 // that no one address takes every workgroup's atomic; a group's last
 // workgroup has its group counter's result before it counts the group.
 __device__ __forceinline__ void pass_end(DevStats* st, int par, unsigned int* clear, unsigned int* conv) {
   if (threadIdx.x != 0) return;
-  const unsigned n_wg = gridDim.x, ng = (n_wg + kPassGroup - 1) / kPassGroup;
-  if (ng > 1 && ng <= (unsigned)kPassGroups) {
-    const unsigned grp = blockIdx.x / kPassGroup;
-    const unsigned members = min((unsigned)kPassGroup, n_wg - grp * kPassGroup);
+  const unsigned n_wg = gridDim.x;
+  const unsigned size = max((unsigned)kPassGroup, (n_wg + kPassGroups - 1) / kPassGroups);
+  const unsigned ng = (n_wg + size - 1) / size;
+  if (ng > 1) {
+    const unsigned grp = blockIdx.x / size;
+    const unsigned members = min(size, n_wg - grp * size);
     unsigned int* gc = &st->pass_grp[grp * kPassStride];
     if (atomicAdd(gc, 1u) + 1 != members) return;
     atomicExch(gc, 0u);  // rearmed for the next pass
