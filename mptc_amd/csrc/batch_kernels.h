@@ -88,32 +88,29 @@ struct DevStats {
 };
 
 // The pruning bound's table of an index word (prune_kernels.h).
-// Per index word: byte masks of groups 0..2 over the four 4-pixel chunks and
-// 1 / (pixels per group) for groups 0..3 (0 for an empty group).
 struct BoundTab {
-  uint4 m0, m1, m2;
-  float4 inv;
+  uint4 w;   // three times the pixel's weight of the first endpoint (0..3), a byte per pixel, as BoundBlk's channels
+  float4 k;  // sum b^2, -2 sum ab, sum a^2, each / (sum a^2 sum b^2 - (sum ab)^2); the rounding slack
 };
 
 __device__ __forceinline__ BoundTab bound_table(uint32_t c) {
-  uint32_t m[3][4];
-  uint32_t n[3] = {0u, 0u, 0u};
+  uint32_t w[4], aa = 0, sa = 0, n23 = 0;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const uint32_t x = spread_indices(c, j);
-#pragma unroll
-    for (int g = 0; g < 3; ++g) {
-      m[g][j] = byte_gather(1u << (8 * g), x);  // 1 in byte n where pixel 4j+n has index g
-      n[g] = __builtin_amdgcn_udot4(m[g][j], 0x01010101u, n[g], false);
-    }
+    w[j] = byte_gather(0x01020003u, x);  // index 0..3 -> 3, 0, 2, 1
+    aa = __builtin_amdgcn_udot4(w[j], w[j], aa, false);
+    sa = __builtin_amdgcn_udot4(w[j], 0x01010101u, sa, false);
+    n23 += (uint32_t)__popc(x & 0x02020202u);
   }
-  const uint32_t n3 = 16u - n[0] - n[1] - n[2];
+  const int bb = 144 - 6 * (int)sa + (int)aa, ab = 3 * (int)sa - (int)aa, det = (int)aa * bb - ab * ab;
+  // slack: the largest norm of the palette's rounding against a line, at its best common shift s
+  const float s = fminf(1.0f / 3.0f, (float)n23 * (1.0f / 24.0f)), r = fmaxf(s, 2.0f / 3.0f - s);
+  const float eta = sqrtf(3.0f * ((float)(16u - n23) * s * s + (float)n23 * r * r)) + 0.001f;
   BoundTab t;
-  t.m0 = make_uint4(m[0][0], m[0][1], m[0][2], m[0][3]);
-  t.m1 = make_uint4(m[1][0], m[1][1], m[1][2], m[1][3]);
-  t.m2 = make_uint4(m[2][0], m[2][1], m[2][2], m[2][3]);
-  t.inv = make_float4(n[0] ? 1.0f / (float)n[0] : 0.0f, n[1] ? 1.0f / (float)n[1] : 0.0f,
-                      n[2] ? 1.0f / (float)n[2] : 0.0f, n3 ? 1.0f / (float)n3 : 0.0f);
+  t.w = make_uint4(w[0], w[1], w[2], w[3]);
+  const float inv = det ? 1.0f / (float)det : 0.0f;  // one index value: never pruned
+  t.k = make_float4((float)bb * inv, (float)(-2 * ab) * inv, (float)aa * inv, det ? eta : 1e9f);
   return t;
 }
 
