@@ -58,8 +58,8 @@ typedef struct {
   int32_t use_graph;  /* replay the step as captured HIP graphs */
   int32_t win_chunks; /* window tile: the 2S window rows of a block are split into
                          this many runs scanned by separate waves, 1..8 */
-  int32_t prune;      /* 1: for S <= 8 and thresholds 0..4, evaluate exactly only the
-                         candidates an error lower bound cannot rule out (same output);
+  int32_t prune;      /* 1: for thresholds 0..4, evaluate exactly only the candidates an
+                         error lower bound cannot rule out (same output);
                          0: evaluate every candidate */
   int32_t itile_w;    /* intra fixpoint passes: 8, 16, 32 or 64: a wave settles the reuse
                          chains inside a tile of itile_w x 64/itile_w blocks per pass;

@@ -83,6 +83,7 @@ struct DevStats {
   unsigned int n_changed[2];             // length of the changed-word list, by pass parity
   unsigned int pass_done;                // workgroups of the running fixpoint pass that finished
   unsigned int skip_tile;                // the last pass was tile-resolved (k_intra_tile_pass)
+  unsigned int n_need;                   // blocks on the list of k_need_list
   unsigned int wave_ticket, wave_done, wave_fail;  // k_intra_wave: rows taken, rows finished, a row gave up
   unsigned int pass_grp[kPassGroups * kPassStride];  // pass_end's group counters
 };
@@ -306,6 +307,12 @@ __device__ __forceinline__ void combine_chunks(const uint4* __restrict__ summ, s
   ret = m;
 }
 
+// Clears n 16-byte vectors (the passing sets above S = 8).
+__global__ void __launch_bounds__(256) k_zero16(uint4* __restrict__ p, size_t n) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+    p[i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
 __global__ void __launch_bounds__(256) k_fill_sid(const FrameDev* __restrict__ fr, int n_frames, uint8_t* __restrict__ sid) {
   const int f = blockIdx.y;
   if (f >= n_frames) return;
@@ -443,8 +450,8 @@ __global__ void __launch_bounds__(256) k_intra_prep(const FrameDev* __restrict__
   dirty[g] = 0;
   const CandTab t = cand_table(w);
   ctab[g] = make_float4(t.asq, t.bsq, t.ab, t.f);
-  if (cbt) {  // the pruned intra search: bound table of the word, passing set empty
-    cbt[g] = bound_table(w);
+  if (cbt) cbt[g] = bound_table(w);  // the pruned intra search: bound table of the word
+  if (pm4) {                          // and, up to S = 8, its passing set cleared
     pm4[2 * g] = make_uint4(0u, 0u, 0u, 0u);
     pm4[2 * g + 1] = make_uint4(0u, 0u, 0u, 0u);
   }
@@ -542,28 +549,27 @@ __device__ __forceinline__ Fold fold_passing(const uint2* __restrict__ E4, size_
   return fd;
 }
 
-// Passing sets: for windows of at most 256 positions (S <= 8), bit p % 32 of
-// word p / 32 of pm[8 g .. 8 g + 7] is set exactly when block g's delta at
-// position p passes (valid, <= thr).  Folding a block then reads its 32 bytes
-// of set and the few passing deltas instead of all of its E.  Where a block
-// keeps a passing set, E holds only its passing deltas (the pruned search
+// Passing sets: bit p % 32 of word p / 32 of block g's pass_words(S) words of
+// pm is set exactly when its delta at position p passes (valid, <= thr).
+// Folding a block then reads its set (32 bytes at S <= 8, 512 at S = 32) and
+// the few passing deltas instead of all of its E (8 KB at S = 32).  Where a
+// block keeps a passing set, E holds only its passing deltas (the pruned search
 // writes only groups of four with a passing one, the passes only passing
 // values); an entry whose bit is clear is not read.
-constexpr int kPassWords = 8;
+constexpr int kPassWords = 8;  // of windows up to S = 8
+__host__ __device__ constexpr int pass_words(int S) {
+  return S <= 8 ? kPassWords : (4 * S * S + 127) / 128 * 4;  // whole 16-byte vectors
+}
 
 __device__ __forceinline__ Fold fold_passing_set(const uint32_t* __restrict__ pm, const uint2* __restrict__ E4,
                                                  size_t nbs, int g, int S) {
-  const int W2 = 2 * S;
-  const uint4* p4 = reinterpret_cast<const uint4*>(pm + (size_t)g * kPassWords);
-  const uint4 a = p4[0], b = p4[1];
-  const uint32_t m[kPassWords] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  const int W2 = 2 * S, n4 = pass_words(S) / 4;
+  const uint4* p4 = reinterpret_cast<const uint4*>(pm) + (size_t)g * n4;
   Fold fd;
   int row = -1;
-#pragma unroll
-  for (int w = 0; w < kPassWords; ++w) {
-    uint32_t mw = m[w];
+  auto word = [&](uint32_t mw, int p0) {
     while (mw != 0u) {  // set bits in increasing position: scan order
-      const int pos = 32 * w + __builtin_ctz(mw);
+      const int pos = p0 + __builtin_ctz(mw);
       mw &= mw - 1u;
       const int e = e_at(E4[(size_t)(pos >> 2) * nbs + g], pos & 3);
       const int r = pos / W2;
@@ -573,26 +579,85 @@ __device__ __forceinline__ Fold fold_passing_set(const uint32_t* __restrict__ pm
       }
       fd.step(e, pos);
     }
+  };
+  for (int i = 0; i < n4; i += 2) {  // n4 is 2, or larger and read two at a time
+    const uint4 a = p4[i], b = i + 1 < n4 ? p4[i + 1] : make_uint4(0u, 0u, 0u, 0u);
+    const uint32_t m[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int w = 0; w < 8; ++w) word(m[w], 128 * i + 32 * w);
   }
   return fd;
 }
 
+// The blocks that search the intra window, for k_intra_dense<true>: 4,096
+// blocks a workgroup, so that few workgroups queue on the list's counter.
+constexpr int kNeedPer = 16;
+__global__ void __launch_bounds__(256) k_need_list(const uint8_t* __restrict__ need, int total, int* __restrict__ list,
+                                                   DevStats* __restrict__ st) {
+  __shared__ unsigned int s_n;
+  __shared__ unsigned int s_at;
+  const int g0 = blockIdx.x * 256 * kNeedPer + threadIdx.x, lane = (int)(threadIdx.x & 63);
+  if (threadIdx.x == 0) s_n = 0;
+  __syncthreads();
+  uint32_t mine = 0;
+  for (int u = 0; u < kNeedPer; ++u) {
+    const int g = g0 + 256 * u;
+    mine |= (g < total && need[g] != 0 ? 1u : 0u) << u;
+  }
+  unsigned int at[kNeedPer];
+#pragma unroll
+  for (int u = 0; u < kNeedPer; ++u) {
+    const unsigned long long m = __ballot((mine >> u) & 1u);
+    unsigned int off = 0;
+    if (m && lane == 0) off = atomicAdd(&s_n, (unsigned int)__popcll(m));
+    at[u] = __shfl(off, 0) + (unsigned int)__popcll(m & ((1ull << lane) - 1));
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 && s_n) s_at = atomicAdd(&st->n_need, s_n);
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kNeedPer; ++u)
+    if ((mine >> u) & 1u) list[s_at + at[u]] = g0 + 256 * u;
+}
+
+// Every intra candidate of every searching block: lane per block, a wave tile's
+// blocks, or (kList) 64 of the list's.  In inter frames at thresholds above 4
+// few blocks search (1080p, threshold 8: 5 %) and hardly a tile has none, so a
+// lane per searching block does a twentieth of the work.
+template <bool kList>
 __global__ void __launch_bounds__(256) k_intra_dense(const FrameDev* __restrict__ fr, const uint8_t* __restrict__ tsid,
                                                      int n_wtiles, int tw, int n_chunks, int S,
                                                      const uint64_t* __restrict__ own, const uint8_t* __restrict__ need,
                                                      const uint32_t* __restrict__ cw, const float4* __restrict__ ctab,
                                                      const int* __restrict__ orig, uint2* __restrict__ E4, size_t nbs,
                                                      uint4* __restrict__ summ, size_t sstride,
-                                                     DevStats* __restrict__ st) {
+                                                     DevStats* __restrict__ st, const int* __restrict__ list,
+                                                     const uint8_t* __restrict__ sid) {
   __shared__ uint8_t s_snap[512];
   __shared__ float2 s_ab[4];
   __shared__ unsigned long long s_acc;
-  load_lds_tables(s_snap, s_ab);
   int f = 0, bx = 0, by = 0, g = 0, chunk = 0;
+  bool in;
+  if (kList) {
+    const unsigned n = st->n_need, w0 = blockIdx.x * (blockDim.x >> 6);
+    if (w0 / n_chunks * 64 >= n) return;  // workgroup-uniform
+    const unsigned w = w0 + (threadIdx.x >> 6), i = w / n_chunks * 64 + (threadIdx.x & 63);
+    chunk = (int)(w % n_chunks);
+    in = i < n;
+    if (in) {
+      g = list[i];
+      f = sid[g];
+      const int k = g - fr[f].base;
+      bx = k % fr[f].bw;
+      by = k / fr[f].bw;
+    }
+  } else {
+    in = tile_block(fr, tsid, n_wtiles, tw, n_chunks, f, bx, by, chunk);
+    if (in) g = fr[f].base + by * fr[f].bw + bx;
+  }
+  load_lds_tables(s_snap, s_ab);
   unsigned long long n_cand = 0;
-  const bool in = tile_block(fr, tsid, n_wtiles, tw, n_chunks, f, bx, by, chunk);
-  if (in) g = fr[f].base + by * fr[f].bw + bx;
-  if (in && need[g]) {
+  if (in && (kList || need[g])) {
     const FrameDev& d = fr[f];
     const int bw = d.bw, base = d.base;
     BlockPx px;
@@ -696,7 +761,7 @@ __device__ __forceinline__ unsigned long long reeval_items(
     size_t nbs, uint32_t* __restrict__ dirty, const int* __restrict__ orig, const uint64_t* __restrict__ dec,
     uint32_t* __restrict__ pm, const uint8_t* s_snap, const float2* s_ab, size_t w0, size_t stride,
     int skip_tw_log) {
-  const int W2 = 2 * S, slots = W2 * W2;
+  const int W2 = 2 * S, slots = W2 * W2, pw = pass_words(S);
   const size_t total = (size_t)n_chg * slots;
   unsigned long long n_eval = 0;
   int16_t* E = reinterpret_cast<int16_t*>(E4);
@@ -741,7 +806,7 @@ __device__ __forceinline__ unsigned long long reeval_items(
     bool passes_old;
     int16_t old;
     if (pm) {  // E is kept only where the passing set has the position
-      passes_old = (pm[(size_t)k * kPassWords + (s >> 5)] >> (s & 31)) & 1u;
+      passes_old = (pm[(size_t)k * pw + (s >> 5)] >> (s & 31)) & 1u;
       old = passes_old ? *slot : kNoCand;
       if (passes_new && old != ev) *slot = ev;
     } else {
@@ -752,7 +817,7 @@ __device__ __forceinline__ unsigned long long reeval_items(
     if ((old != ev && (passes_old || passes_new)) || is_sel) dirty[k] = 1u;
     // one work item per (block, position) in a pass: bits of a word flip
     // concurrently only for different positions
-    if (pm && passes_old != passes_new) atomicXor(&pm[(size_t)k * kPassWords + (s >> 5)], 1u << (s & 31));
+    if (pm && passes_old != passes_new) atomicXor(&pm[(size_t)k * pw + (s >> 5)], 1u << (s & 31));
   }
   return n_eval;
 }
@@ -889,7 +954,7 @@ __global__ void __launch_bounds__(256) k_intra_tile_pass(
   if (blockIdx.x == 0 && threadIdx.x == 0) st->skip_tile = 1u;  // read by the next pass's k_intra_reeval
   const int wv = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
   const int lane = (int)(threadIdx.x & 63);
-  const int W2 = 2 * S;
+  const int W2 = 2 * S, pw = pass_words(S);
   int16_t* E = reinterpret_cast<int16_t*>(E4);
   unsigned long long n_eval = 0;
   bool changed = false;
@@ -983,7 +1048,7 @@ __global__ void __launch_bounds__(256) k_intra_tile_pass(
         bool passes_old;
         int16_t old;
         if (pm) {  // E is kept only where the passing set has the position
-          passes_old = (pm[(size_t)g * kPassWords + (s >> 5)] >> (s & 31)) & 1u;
+          passes_old = (pm[(size_t)g * pw + (s >> 5)] >> (s & 31)) & 1u;
           old = passes_old ? *slot : kNoCand;
           if (passes_new && old != ev) *slot = ev;
         } else {
@@ -994,7 +1059,7 @@ __global__ void __launch_bounds__(256) k_intra_tile_pass(
         const bool is_sel = dec_acc(dc) && (W2 - 1 - (int)((dc >> 40) & 0xFF)) * W2 +
                                                    (W2 - 1 - (int)((dc >> 32) & 0xFF)) == s;
         if ((old != ev && (passes_old || passes_new)) || is_sel) redo = true;
-        if (pm && passes_old != passes_new) pm[(size_t)g * kPassWords + (s >> 5)] ^= 1u << (s & 31);
+        if (pm && passes_old != passes_new) pm[(size_t)g * pw + (s >> 5)] ^= 1u << (s & 31);
       }
     }
     changed = inside && cur != start;

@@ -235,7 +235,7 @@ struct mptc_ctx {
   int16_t* d_prop = nullptr;    // intra proposals, kMaxTopK per block
   // pruned exhaustive search (prune_kernels.h), allocated on first use
   BoundTab *d_rbt = nullptr, *d_cbt = nullptr;  // bound tables of reference / current words
-  uint32_t* d_pm = nullptr;                      // passing sets of the intra windows (kPassWords per block)
+  uint32_t* d_pm = nullptr;                      // passing sets of the intra windows (pass_words(alloc_S) per block)
   bool record = false;          // exhaustive steps record acceptance masks
   bool last_recorded = false;   // the last step did
   uint16_t* d_amask[2] = {nullptr, nullptr};  // inter, intra: 16 rows of 16 offset bits per block
@@ -523,20 +523,25 @@ int prepare_batch(mptc_ctx* c, hipStream_t s, int n, const FrameIn* in) {
   return MPTC_OK;
 }
 
-// The pruned exhaustive search applies to small windows and thresholds, where
-// the bound rules out most candidates (thresholds 0..kPruneMaxThr).
+// The pruned exhaustive searches (prune_kernels.h) take thresholds 0 to
+// kPruneMaxThr, any search area.  Above, the bound leaves most candidates: at
+// threshold 8 it is 91 % of them, and in the inter search still 86 % (the
+// previous frame's words are the widely reusable ones) when each lane prunes
+// against the smallest delta it and the window's other chunks have found; twelve
+// streams, threshold 8: 5.5 ms so, 4.4 with every candidate evaluated.
 constexpr int kPruneMaxThr = 4;
 
 bool use_prune(const mptc_ctx* c) {
-  return c->tune.prune && c->mode == MPTC_SEARCH_EXHAUSTIVE && !c->record && c->cfg.search_area <= kPruneMaxS &&
-         c->cfg.err_threshold >= 0 && c->cfg.err_threshold <= kPruneMaxThr;
+  return c->tune.prune && c->mode == MPTC_SEARCH_EXHAUSTIVE && !c->record && c->cfg.err_threshold >= 0 &&
+         c->cfg.err_threshold <= kPruneMaxThr;
 }
 
 int prune_ensure(mptc_ctx* c) {
   if (c->d_rbt) return MPTC_OK;
   const size_t nb = (size_t)c->max_total;
   int rc;
-  if ((rc = dalloc(&c->d_rbt, nb)) || (rc = dalloc(&c->d_cbt, nb)) || (rc = dalloc(&c->d_pm, nb * kPassWords)))
+  if ((rc = dalloc(&c->d_rbt, nb)) || (rc = dalloc(&c->d_cbt, nb)) ||
+      (rc = dalloc(&c->d_pm, nb * pass_words(c->alloc_S))))
     return rc;
   return MPTC_OK;
 }
@@ -608,7 +613,7 @@ int lintra_pass_q(mptc_ctx* c, hipStream_t s, int par, int first, bool report) {
 //    8 23 / 4.8, 32 40 / 4.3; S = 32: 8 288 / 25, 32 770 / 12;
 //  - above S = 16, where a window may hold more distinct words than there are
 //    ids (1080p, S = 32: up to 2,100 at threshold 4, 800 at 8), from 8 on.
-constexpr int kWaveMinThr = 5, kWaveWideS = 16, kWaveWideThr = 8;
+constexpr int kWaveMinThr = kPruneMaxThr + 1, kWaveWideS = 16, kWaveWideThr = 8;
 
 bool use_wave(const mptc_ctx* c) {
   const int S = c->cfg.search_area;
@@ -635,7 +640,8 @@ int queue_intra_prep(mptc_ctx* c, hipStream_t s, bool prune, bool wave, const ui
     hipLaunchKernelGGL(k_intra_prep, dim3(grid_for(total, wg)), dim3(wg), 0, s, c->d_fr, c->d_sid, total, c->d_own,
                        c->d_inter, c->d_need, c->d_cw, lrn ? nullptr : c->d_ctab, lrn ? nullptr : c->d_dirty,
                        lrn ? nullptr : c->d_orig, prune ? c->d_cbt : nullptr,
-                       prune ? reinterpret_cast<uint4*>(c->d_pm) : nullptr, chunks_for(S, c->tune.win_chunks), S,
+                       prune && S <= 8 ? reinterpret_cast<uint4*>(c->d_pm) : nullptr,
+                       chunks_for(S, c->tune.win_chunks), S,
                        c->cfg.err_threshold, c->d_rw, inter_summ, c->nbs, orig_ready, wave ? c->d_fin : nullptr, c->d_summ);
   });
 }
@@ -653,7 +659,7 @@ int queue_prefix(mptc_ctx* c, hipStream_t s, bool fit, bool wave) {
                        (c->mode == MPTC_SEARCH_LEARNED && !c->net[MPTC_NET_INTRA].use_prior));
   bool x_done = want_x;
   bool prep_done = false;  // need and the starting intra words already set
-  const bool prune = use_prune(c) && !wave;
+  const bool prune = use_prune(c);  // (no wave then: its thresholds are higher)
   if ((rc = launch(c, s, KF_FIT, [&] {
          const int n_st = (int)(sizeof(DevStats) / 4);
          hipLaunchKernelGGL(k_block_prep, dim3(grid_for(std::max(total, n_st + c->n_tiles), wg)), dim3(wg), 0, s,
@@ -708,7 +714,12 @@ int queue_prefix(mptc_ctx* c, hipStream_t s, bool fit, bool wave) {
     if ((rc = proposals_q(c, s, MPTC_NET_INTRA, c->d_need, c->d_prop, x_done))) return rc;
     return lintra_pass_q(c, s, 0, 1, false);
   }
-  if (prune) {  // bound tables and cleared passing sets from k_intra_prep
+  if (prune) {  // bound tables and (up to S = 8) cleared passing sets from k_intra_prep
+    if (S > 8 && (rc = launch(c, s, KF_PREP, [&] {
+          hipLaunchKernelGGL(k_zero16, dim3(2048), dim3(256), 0, s, reinterpret_cast<uint4*>(c->d_pm),
+                             (size_t)total * pass_words(S) / 4);
+        })))
+      return rc;
     // with 1, 2 or 4 chunks every tile's chunks are waves of one workgroup,
     // and the search also takes the intra decisions (k_fold_intra's work)
     const int fold = 4 % K == 0 ? 1 : 0;
@@ -729,10 +740,17 @@ int queue_prefix(mptc_ctx* c, hipStream_t s, bool fit, bool wave) {
                          c->d_stats);
     });
   }
+  // a batch with inter frames above the pruned thresholds: a lane per searching
+  // block (listed in d_chg, which the combine fills afterwards)
+  const bool listed = c->any_inter && thr > kPruneMaxThr;
   if ((rc = launch(c, s, KF_DENSE, [&] {
-         hipLaunchKernelGGL(k_intra_dense, dim3(gwk), dim3(wg), 0, s, c->d_fr, c->d_tsid, c->n_wtiles, tw, K, S,
-                            c->d_own, c->d_need, c->d_cw, c->d_ctab, c->d_orig, c->d_E, c->nbs, c->d_summ, c->nbs,
-                            c->d_stats);
+         if (listed)
+           hipLaunchKernelGGL(k_need_list, dim3(grid_for(total, 256 * kNeedPer)), dim3(256), 0, s, c->d_need, total,
+                              c->d_chg, c->d_stats);
+         auto kern = listed ? k_intra_dense<true> : k_intra_dense<false>;
+         hipLaunchKernelGGL(kern, dim3(listed ? grid_for((total + 63) / 64 * K * 64, wg) : gwk), dim3(wg), 0, s,
+                            c->d_fr, c->d_tsid, c->n_wtiles, tw, K, S, c->d_own, c->d_need, c->d_cw, c->d_ctab,
+                            c->d_orig, c->d_E, c->nbs, c->d_summ, c->nbs, c->d_stats, c->d_chg, c->d_sid);
        })))
     return rc;
   if ((rc = launch(c, s, KF_INTRA_COMBINE, [&] {

@@ -56,8 +56,6 @@
 namespace mptc {
 
 constexpr int16_t kPruned = 32766;  // E value of a candidate proved not to pass
-constexpr int kPruneMaxS = 8;       // window positions of one batch fit the LDS list
-static_assert(4 * kPruneMaxS * kPruneMaxS <= 32 * kPassWords, "a passing set holds every window position");
 
 // Pixel side of the bound for one block.
 struct BoundBlk {
@@ -129,7 +127,7 @@ constexpr int kFoldWords = 8;    // LDS words of an inter lane's fold: ChunkFold
 
 // An inter lane's ChunkFold lives in LDS between the (rare) batches that
 // have passing deltas, so that it holds no registers through the rest.  Its
-// fields fit 16 bits: positions < 1024, rows < 64, and min_val is a passing
+// fields fit 16 bits: positions < 15,876, rows < 126, and min_val is a passing
 // delta (<= thr) or the initial "none" (stored as kNoCand).
 __device__ __forceinline__ void cf_load(int16_t (*s)[64], int lane, ChunkFold& cf, int& row) {
   cf.first_le0 = s[0][lane];
@@ -317,7 +315,7 @@ __global__ void __launch_bounds__(256) k_pruned_search(const FrameDev* __restric
       }
       if (bits) {  // rare; the batch's 16 bits may straddle two words, which other chunks' waves share
         const int sh = pb & 31;
-        uint32_t* wp = pm + (size_t)g * kPassWords + (pb >> 5);
+        uint32_t* wp = pm + (size_t)g * pass_words(S) + (pb >> 5);
         atomicOr(wp, bits << sh);
         if (sh > 16 && (bits >> (32 - sh)) != 0u) atomicOr(wp + 1, bits >> (32 - sh));
       }

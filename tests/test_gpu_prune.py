@@ -1,0 +1,54 @@
+"""Pruned searches beyond S = 8 (thresholds to 4) and the listed intra search of
+inter frames (thresholds above) against the CPU oracle."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from mptc_amd.workloads import SynthCfg
+from tests.helpers import compare_results
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def enc():
+    from mptc_amd import lib
+    e = lib.Encoder(320, 320, search_area=63, err_threshold=0)
+    yield e
+    e.close()
+
+
+# windows whose positions fill no whole vector, chunk or batch; sizes under the window; one set word to several
+@pytest.mark.parametrize("w,h,S,thr", [(100, 60, 9, 0), (100, 60, 9, 3), (132, 68, 11, 4), (160, 96, 16, 0), (160, 96, 16, 4),
+                                       (140, 80, 17, 2), (200, 120, 32, 0), (200, 120, 32, 4), (96, 64, 63, 1),
+                                       (4, 100, 12, 2), (200, 4, 12, 2), (160, 96, 8, 8), (160, 96, 3, 9), (100, 60, 5, 300),
+                                       (160, 96, 16, 8), (200, 120, 32, 16), (160, 96, 33, 8), (36, 36, 8, 30000)])
+def test_searches_match_oracle(enc, orc, w, h, S, thr):
+    print(f"{w}x{h} S={S} thr={thr}", flush=True)
+    frames = orc.synth_frames(SynthCfg(w, h, w + S, 5, 1, 3, 8, 0), 3)
+    enc.set_params(S, thr)
+    got = enc.encode_sequence(frames, 8)
+    st = enc.stats()
+    want = orc.encode_sequence(frames, S, thr, 8)
+    for f, (a, b) in enumerate(zip(got, want)):
+        compare_results(a, b, f"frame {f}")
+        assert np.array_equal(a["kind"], b["kind"])
+    assert (st["exact_inter_candidates"] > 0) == (thr <= 4)
+    assert st["exact_inter_candidates"] <= st["inter_candidates"]
+
+
+@pytest.mark.parametrize("prune", [0, 1])
+def test_flat_and_saturated_blocks(enc, orc, prune):
+    """Blocks of one colour (equal endpoints: nothing is pruned for them), of two
+    extreme colours, and reference words of one index value."""
+    rng = np.random.default_rng(8)
+    a = np.repeat(np.repeat(rng.choice([0, 7, 255], (30, 40, 3)), 4, 0), 4, 1).astype(np.uint8)
+    b = np.where(rng.random((120, 160, 3)) < 0.3, 255 - a, a).astype(np.uint8)
+    frames = np.stack([a, b, np.roll(a, 4, 1)])
+    enc.set_tuning(prune=prune)
+    for S, thr in ((8, 0), (8, 9), (12, 2)):
+        enc.set_params(S, thr)
+        for f, (x, y) in enumerate(zip(enc.encode_sequence(frames, 8), orc.encode_sequence(frames, S, thr, 8))):
+            compare_results(x, y, f"S={S} thr={thr} frame {f}")
+    enc.set_tuning()
