@@ -533,7 +533,7 @@ constexpr int kPruneMaxThr = 4;
 
 bool use_prune(const mptc_ctx* c) {
   return c->tune.prune && c->mode == MPTC_SEARCH_EXHAUSTIVE && !c->record && c->cfg.err_threshold >= 0 &&
-         c->cfg.err_threshold <= kPruneMaxThr;
+         c->cfg.err_threshold <= kPruneMaxThr && c->total <= 1 << 27;  // 32-bit offsets of the words' tables
 }
 
 int prune_ensure(mptc_ctx* c) {

@@ -7,7 +7,7 @@
 // first passing candidate (scan order) the others can only raise the running
 // minimum, which that candidate then undercuts; after it they can never update
 // it (codec/dxt_image.cpp:697-708).  So a candidate proved non-passing may be
-// recorded as any non-passing value (kPruned) without changing the decision.
+// recorded as not passing without changing the decision.
 //
 // The bound.  A valid candidate's palette is two endpoints and the points a
 // third and two thirds between them, rounded down: q_i = a_i e1 + (1 - a_i) e2 -
@@ -31,9 +31,9 @@
 // form too, unless its endpoints are in the order that means a three-colour
 // palette; such a block prunes nothing.
 //
-//   k_pruned_search wave tiles as the search kernels; per position the bound,
-//                   non-passing -> kPruned; the wave's survivors are compacted
-//                   in LDS and evaluated exactly, 64 per round.  Inter: the
+//   k_pruned_search wave tiles as the search kernels; per position the bound;
+//                   the wave's survivors are compacted in LDS and evaluated
+//                   exactly, 64 per round.  Inter: the
 //                   chunk summaries of the selection rule (as k_inter, then
 //                   inter_decision in k_intra_prep); intra: E for the
 //                   fixpoint passes
@@ -55,7 +55,6 @@
 
 namespace mptc {
 
-constexpr int16_t kPruned = 32766;  // E value of a candidate proved not to pass
 
 // Pixel side of the bound for one block.
 struct BoundBlk {
@@ -156,9 +155,15 @@ __device__ __forceinline__ void cf_store(int16_t (*s)[64], int lane, const Chunk
 // kernels.  Per batch of kPruneBatch positions each lane bounds its block's
 // candidates; the survivors of the whole wave are compacted in LDS and
 // evaluated exactly 64 at a time, a lane taking any block's survivor (the
-// pixel side of the wave's 64 blocks is kept in LDS).  Each position's value
-// is the exact delta of a survivor, kPruned for a pruned and kNoCand for an
-// absent position.  Intra: the values go to E.  Inter: each lane folds its
+// pixel side of the wave's 64 blocks is kept in LDS).  Passing survivors leave
+// their delta and a bit of their block's batch.  The bounds are what the time
+// goes to, so their loop holds little else: 52 vector instructions a position
+// where it had 97 (the window row's part of the address and of the edge test is
+// kept for the row, positions that do not pass are not recorded, the bounded
+// positions are counted from the window's shape), and two positions' tables are
+// requested together (one at a time behind its edge test: 17.5 ms).  A
+// 3840x2160 inter frame of S = 32 at threshold 0: 14.7 -> 13.7 ms.
+// Intra: the values go to E.  Inter: each lane folds its
 // chunk's passing values in scan order into the chunk summary summ[chunk][g]
 // of the dense inter kernel (for thr >= 0 the selection depends only on the
 // passing deltas, and a row without one leaves a summary as it is).
@@ -177,9 +182,9 @@ __global__ void __launch_bounds__(256) k_pruned_search(const FrameDev* __restric
   __shared__ uint8_t s_snap[512];
   __shared__ float2 s_ab[4];
   __shared__ uint32_t s_blk[4][kPackedBlk][64];      // [wave][field][lane]
-  __shared__ int16_t s_e[4][kPruneBatch][64];        // the batch's E values, [wave][position][lane]
+  __shared__ int16_t s_e[4][kPruneBatch][64];        // the batch's passing deltas, [wave][position][lane]
   __shared__ uint16_t s_list[4][kPruneBatch * 64 + 64];  // survivors: lane | position << 6; + per-lane dummies
-  __shared__ uint8_t s_pass[4][64];                      // inter: the lane's batch holds a passing delta
+  __shared__ uint32_t s_pass[4][64];                     // the lane's passing positions of the batch
   __shared__ int16_t s_cf[4][kFoldWords][64];            // inter: each lane's ChunkFold state and row
   __shared__ unsigned long long s_acc;
   __shared__ unsigned int s_base;
@@ -215,7 +220,7 @@ __global__ void __launch_bounds__(256) k_pruned_search(const FrameDev* __restric
     s_blk[wave][13][lane] = (uint32_t)(own[g] >> 32);
     s_blk[wave][14][lane] = (uint32_t)e_own;
   }
-  unsigned long long n_bound = 0, n_exact = 0;
+  unsigned long long n_exact = 0;
   const int W2 = 2 * S, rows = W2 / n_chunks, p0 = chunk * rows * W2, p1 = p0 + rows * W2;
   // (rb, tb): window row and column of the batch's first position, stepped
   // without divisions
@@ -227,6 +232,16 @@ __global__ void __launch_bounds__(256) k_pruned_search(const FrameDev* __restric
   const bool wave_act = __ballot(act) != 0ull;
   // the frame's fields in registers (the loops' stores could otherwise alias them)
   const int fbw = d.bw, fbh = d.bh, fbase = d.base;
+  // window row of the running position: whether the block has it, and its first block in the frame (clamped into it)
+  const char* const ftab = reinterpret_cast<const char*>(btab + fbase);
+  bool row_in = false;
+  int row_at = 0;
+  auto set_row = [&](int r) {
+    const int j = kIntra ? by - r : by - S + r;
+    row_in = act && j >= 0 && j < fbh;
+    row_at = min(max(j, 0), fbh - 1) * fbw;
+  };
+  set_row(rb);
   // inter: the selection rule over the chunk's positions in scan order
   if (!kIntra) {
     ChunkFold cf;
@@ -237,7 +252,7 @@ __global__ void __launch_bounds__(256) k_pruned_search(const FrameDev* __restric
     const int nb = min(kPruneBatch, p1 - pb);  // a multiple of 4
     uint32_t cnt = 0;                          // wave-uniform
     int r = rb, t = tb;
-    if (!kIntra) s_pass[wave][lane] = 0;
+    s_pass[wave][lane] = 0u;
     // the block's bound constants, rebuilt from LDS for each batch so that they
     // hold no registers through the evaluations (zero for lanes that do not
     // search: their bounds are computed and ignored)
@@ -249,23 +264,33 @@ __global__ void __launch_bounds__(256) k_pruned_search(const FrameDev* __restric
       make_bound_blk(c, b);
       b.rl = bound_limit(thr, (int)s_blk[wave][14][lane], line);
     }
-    for (int k = 0; k < nb; ++k) {
-      int j = 0, i = 0;
-      const bool there = act & window_block<kIntra>(r, t, S, bx, by, fbw, fbh, j, i);
-      t = t + 1 == W2 ? 0 : t + 1;
-      r += t == 0 ? 1 : 0;
-      // clamped into the frame: the load is always in bounds
-      const int q = fbase + min(max(j, 0), fbh - 1) * fbw + min(max(i, 0), fbw - 1);
-      const bool pruned = bound_prunes(b, btab[q]);
-      const bool surv = there && !pruned;
-      n_bound += there ? 1u : 0u;
-      const unsigned long long bal = __ballot(surv);
-      // survivors take the next list slots; the others write their lane's dummy slot
-      const uint32_t slot = surv ? cnt + (uint32_t)__popcll(bal & ((1ull << lane) - 1))
-                                 : (uint32_t)(kPruneBatch * 64 + lane);
-      s_list[wave][slot] = (uint16_t)(lane | (k << 6));
-      s_e[wave][k][lane] = (int16_t)(there ? kPruned : kNoCand);  // survivors' entries are replaced below
-      cnt += (uint32_t)__popcll(bal);
+    // two positions a step (rows and batches are of even length): both tables are requested before the first is used
+    for (int k = 0; k < nb; k += 2) {
+      bool there[2];
+      BoundTab tb4[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int i = kIntra ? bx + S - 1 - t - u : bx - S + t + u;
+        const int ic = min(max(i, 0), fbw - 1);  // clamped into the frame: the load is always in bounds
+        there[u] = row_in & (i == ic) & !(kIntra && r == 0 && t + u < S);
+        // 32-bit offset into the frame's tables (use_prune: batches of at most 2^27 blocks)
+        tb4[u] = *reinterpret_cast<const BoundTab*>(ftab + (uint32_t)(row_at + ic) * (uint32_t)sizeof(BoundTab));
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const bool surv = there[u] & !bound_prunes(b, tb4[u]);
+        const unsigned long long bal = __builtin_amdgcn_ballot_w64(surv);
+        // survivors take the next list slots; the others write their lane's dummy slot
+        const uint32_t before = __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, cnt));
+        const uint32_t slot = surv ? before : (uint32_t)(kPruneBatch * 64 + lane);
+        s_list[wave][slot] = (uint16_t)(lane | ((k + u) << 6));
+        cnt += (uint32_t)__popcll(bal);
+      }
+      t += 2;
+      if (t == W2) {
+        t = 0;
+        set_row(++r);
+      }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -291,58 +316,54 @@ __global__ void __launch_bounds__(256) k_pruned_search(const FrameDev* __restric
         const float4 t4 = tabs[q];
         const CandResult res =
             eval_candidate<false, true>(be, words[q], CandTab{t4.x, t4.y, t4.z, t4.w}, s_snap, s_ab);
-        s_e[wave][k][lb] = res.valid ? sat16(res.err) : kNoCand;
-        if (!kIntra && res.valid && res.err <= thr) s_pass[wave][lb] = 1;  // (equal writes may race)
+        if (res.valid && res.err <= thr) {
+          s_e[wave][k][lb] = sat16(res.err);
+          atomicOr(&s_pass[wave][lb], 1u << k);
+        }
         ++n_exact;
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (act && kIntra) {  // intra: E and the passing set, for the fixpoint passes
-      uint32_t bits = 0;  // bit k: position pb + k passes
+    uint32_t bits = act ? s_pass[wave][lane] : 0u;  // bit k: position pb + k passes
+    if (kIntra && bits) {  // E and the passing set, for the fixpoint passes
       for (int k = 0; k < nb; k += 4) {
-        const int16_t e0 = s_e[wave][k][lane], e1 = s_e[wave][k + 1][lane], e2 = s_e[wave][k + 2][lane],
-                      e3 = s_e[wave][k + 3][lane];
-        const uint32_t gb = (uint32_t)((e0 != kNoCand && e0 <= thr) | (e1 != kNoCand && e1 <= thr) << 1 |
-                                       (e2 != kNoCand && e2 <= thr) << 2 | (e3 != kNoCand && e3 <= thr) << 3);
-        if (gb) {  // E is kept only where a delta passes (the passing set says where)
-          const uint32_t lo = (uint32_t)(uint16_t)e0 | ((uint32_t)(uint16_t)e1 << 16);
-          const uint32_t hi = (uint32_t)(uint16_t)e2 | ((uint32_t)(uint16_t)e3 << 16);
+        if ((bits >> k) & 15u) {  // E is kept only where a delta passes (the passing set says where)
+          const uint32_t lo = (uint32_t)(uint16_t)s_e[wave][k][lane] | ((uint32_t)(uint16_t)s_e[wave][k + 1][lane] << 16);
+          const uint32_t hi =
+              (uint32_t)(uint16_t)s_e[wave][k + 2][lane] | ((uint32_t)(uint16_t)s_e[wave][k + 3][lane] << 16);
           E4[(size_t)((pb + k) >> 2) * nbs + g] = make_uint2(lo, hi);
         }
-        bits |= gb << k;
       }
-      if (bits) {  // rare; the batch's 16 bits may straddle two words, which other chunks' waves share
-        const int sh = pb & 31;
-        uint32_t* wp = pm + (size_t)g * pass_words(S) + (pb >> 5);
-        atomicOr(wp, bits << sh);
-        if (sh > 16 && (bits >> (32 - sh)) != 0u) atomicOr(wp + 1, bits >> (32 - sh));
-      }
-    } else if (!kIntra && __ballot(act && s_pass[wave][lane] != 0) != 0ull) {
+      // rare; the batch's 16 bits may straddle two words, which other chunks' waves share
+      const int sh = pb & 31;
+      uint32_t* wp = pm + (size_t)g * pass_words(S) + (pb >> 5);
+      atomicOr(wp, bits << sh);
+      if (sh > 16 && (bits >> (32 - sh)) != 0u) atomicOr(wp + 1, bits >> (32 - sh));
+    } else if (!kIntra && bits) {
       // inter: fold the batch's passing deltas in scan order.  The selection
       // depends only on them (thr >= 0), and a row without one leaves the
       // summary as it is, so the other positions are skipped.
-      if (act && s_pass[wave][lane] != 0) {
-        ChunkFold cf;
-        int cf_row;
-        cf_load(s_cf[wave], lane, cf, cf_row);
-        int rr = rb, tt = tb;
-        for (int k = 0; k < nb; ++k) {
-          const int v = s_e[wave][k][lane];
-          if (v != kNoCand && v <= thr) {
-            if (rr != cf_row) {
-              cf.end_row(cf_row);
-              cf.begin_row();
-              cf_row = rr;
-            }
-            cf.step(v, pb + k, rr);
-          }
-          tt = tt + 1 == W2 ? 0 : tt + 1;
-          rr += tt == 0 ? 1 : 0;
+      ChunkFold cf;
+      int cf_row;
+      cf_load(s_cf[wave], lane, cf, cf_row);
+      int rr = rb, t0 = tb;  // row rr holds positions t0 .. W2 - 1, counted from the batch's first
+      while (bits) {
+        const int k = __builtin_ctz(bits);
+        bits &= bits - 1u;
+        while (t0 + k >= W2) {
+          t0 -= W2;
+          ++rr;
         }
-        cf_store(s_cf[wave], lane, cf, cf_row);
+        if (rr != cf_row) {
+          cf.end_row(cf_row);
+          cf.begin_row();
+          cf_row = rr;
+        }
+        cf.step(s_e[wave][k][lane], pb + k, rr);
       }
+      cf_store(s_cf[wave], lane, cf, cf_row);
     }
     // the next batch overwrites s_e and s_list
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -377,6 +398,13 @@ __global__ void __launch_bounds__(256) k_pruned_search(const FrameDev* __restric
       }
     }
     wg_append(changed, g, chg_list, &st->n_changed[0], &s_base);
+  }
+  // positions bounded: the chunk's window rows and columns inside the frame
+  unsigned long long n_bound = 0;
+  if (act) {
+    const int r0 = chunk * rows, lo = kIntra ? r0 : max(r0, S - by), hi = min(r0 + rows, kIntra ? by + 1 : fbh - by + S);
+    const int left = bx - max(0, bx - S), cols = left + min(fbw, bx + S) - bx;
+    if (hi > lo) n_bound = (unsigned long long)(hi - lo) * cols - (kIntra && lo == 0 ? cols - left : 0);
   }
   wg_count(&s_acc, n_bound, kIntra ? st->intra_cands : st->inter_cands);
   wg_count(&s_acc, n_exact, kIntra ? st->exact_intra : st->exact_inter);

@@ -52,3 +52,21 @@ def test_flat_and_saturated_blocks(enc, orc, prune):
         for f, (x, y) in enumerate(zip(enc.encode_sequence(frames, 8), orc.encode_sequence(frames, S, thr, 8))):
             compare_results(x, y, f"S={S} thr={thr} frame {f}")
     enc.set_tuning()
+
+
+@pytest.mark.parametrize("w,h,S", [(4, 4, 1), (12, 8, 1), (100, 60, 2), (36, 132, 5), (132, 36, 8), (96, 64, 12), (40, 200, 32)])
+def test_bounded_positions_are_the_window_inside_the_frame(enc, orc, w, h, S):
+    """The candidate counts of the pruned searches are those of the plain ones."""
+    frames = orc.synth_frames(SynthCfg(w, h, w + S, 5, 1, 3, 8, 0), 2)
+    bw, bh = w // 4, h // 4
+    window = sum((min(bw, x + S) - max(0, x - S)) * (min(bh, y + S) - max(0, y - S)) for x in range(bw) for y in range(bh))
+    counts = []
+    for prune in (0, 1):
+        enc.set_tuning(prune=prune)
+        enc.set_params(S, 0)
+        enc.encode_sequence(frames, 8)
+        st = enc.stats()
+        counts.append((st["inter_candidates"], st["intra_candidates"]))
+    enc.set_tuning()
+    assert counts[0] == counts[1]
+    assert counts[1][0] in (window, 2 * window)  # of the last frame, or of both where the counts run on
