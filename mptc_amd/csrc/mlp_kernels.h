@@ -86,11 +86,15 @@ __global__ void __launch_bounds__(256) k_net_input(const uint8_t* __restrict__ p
 //      W3T [272][256] (W3 transposed, rows 262..271 zero)  forward, layer 3
 //      W2R [256][256] (W2 as stored)                      dH1 = dH2 W2^T
 //      W3R [256][288] (W3, columns 262..287 zero)          dH2 = dY W3^T
-//  - the batch's activations and output gradients, feature-major (row f
-//    holds feature f of every batch row, row stride ld = the batch rounded up
-//    to 32), bf16: X (64 rows, 48..63 zero), H1, H2, dY (320 rows, 262..319
-//    zero), dH2, dH1 -- the operands of the weight gradients, whose k is the
-//    batch row.
+//  - the batch's activations and output gradients, in blocks of 16 batch rows
+//    (ld = the batch rounded up to 32 holds ld / 16 of them), each
+//    [feature][16 rows], bf16: X (64 features, 48..63 zero), H1, H2, dY (320,
+//    262..319 zero), dH2, dH1 -- the operands of the weight gradients, whose k
+//    is the batch row.  A k_train_rows workgroup writes one whole block (45 KB)
+//    and 16 features' fragments of k_train_wgrad are 512-byte runs; with one
+//    row of all ld batch rows per feature both moved 32 to 64 bytes at a stride
+//    of 2 ld (8 KB at 4,096 rows, the same few memory channels: k_train_wgrad
+//    14.3 us, 8.6 so).
 // ---------------------------------------------------------------------------
 constexpr int kTrW1T = 0;
 constexpr int kTrW2T = kTrW1T + kNetHid * 64;
@@ -100,6 +104,7 @@ constexpr int kTrW3R = kTrW2R + kNetHid * kNetHid;
 constexpr int kTrSize = kTrW3R + kNetHid * 288;  // bf16 elements
 constexpr int kActX = 0, kActH1 = 64, kActH2 = kActH1 + kNetHid, kActDY = kActH2 + kNetHid;
 constexpr int kActDH2 = kActDY + 320, kActDH1 = kActDH2 + kNetHid, kActRows = kActDH1 + kNetHid;  // 1408
+constexpr int kActBlk = kActRows * 16;  // elements of a block of 16 batch rows
 constexpr int kBiasCols = 2 * kNetHid + kNetOut;           // 774: db1, db2, db3 in parameter order
 constexpr long kWgPart = 64L * 256 + 256L * 256 + 256L * 320;  // floats of one split's weight gradients
 constexpr int kWgTiles = 4 + 16 + 20;                      // 64 x 64 tiles of dW1, dW2, dW3
@@ -175,11 +180,12 @@ __device__ __forceinline__ void zero_acc(f32x4_t (&acc)[RT][NJ]) {
 // Epilogue of a 256-wide layer: wave columns c0 + 16 j + (lane % 16), rows
 // 16 i + (lane / 16) * 4 + t.  H = relu(acc + bias) (forward, mask null) or
 // acc * [mask > 0] (backward); bf16 to the LDS rows sO (when non-null) and as
-// 4 consecutive rows of one feature to gO (feature-major, row stride ld);
+// 4 consecutive rows of one feature to gO (the layer's features in the
+// workgroup's first block);
 // with cpo, the fp32 column sums over the workgroup's rows go to cpo[col].
 template <int RT>
 __device__ __forceinline__ void layer_out(const f32x4_t (&acc)[RT][4], int c0, int lane, const float* __restrict__ bias,
-                                          const uint16_t* mask, uint16_t* sO, uint16_t* __restrict__ gO, int ld,
+                                          const uint16_t* mask, uint16_t* sO, uint16_t* __restrict__ gO,
                                           float* __restrict__ cpo) {
   constexpr int LH = kNetHid + 8;
   const int col_in = lane & 15, rq = (lane >> 4) * 4;
@@ -205,7 +211,7 @@ __device__ __forceinline__ void layer_out(const f32x4_t (&acc)[RT][4], int c0, i
         sO[(r + 2) * LH + col] = (uint16_t)p23;
         sO[(r + 3) * LH + col] = (uint16_t)(p23 >> 16);
       }
-      *reinterpret_cast<uint2*>(gO + (long)col * ld + 16 * i + rq) = make_uint2(p01, p23);
+      *reinterpret_cast<uint2*>(gO + i * kActBlk + col * 16 + rq) = make_uint2(p01, p23);
     }
     if (cpo) {
       cs += __shfl_xor(cs, 16);
@@ -218,7 +224,7 @@ __device__ __forceinline__ void layer_out(const f32x4_t (&acc)[RT][4], int c0, i
 // One workgroup (4 waves) per 16 RT batch rows: the forward pass (H1, H2,
 // logits and seeds), the loss and dY = d(mean loss)/dY, and the backward
 // products dH2 = (dY W3^T) * [H2 > 0], dH1 = (dH2 W2^T) * [H1 > 0], all
-// held in LDS; the weight-gradient operands go out feature-major (act) and
+// held in LDS; the weight-gradient operands go out as blocks of act and
 // the bias gradients as this workgroup's column sums of dH1, dH2, dY in fp32
 // (colpart[wg][774]).  Wave w computes columns 64 w .. 64 w + 63 of each
 // 256-wide layer (RT x 4 MFMA tiles) and column tiles w, w + 4, ... of the 17
@@ -235,7 +241,7 @@ __device__ __forceinline__ void layer_out(const f32x4_t (&acc)[RT][4], int c0, i
 // takes its 4 RT rows at once (64 / (4 RT) lanes per row).  The batch's mean
 // loss is added to *loss (one atomic per workgroup).
 template <int RT>
-__global__ void __launch_bounds__(256) k_train_rows(int n, int ld, const uint8_t* __restrict__ px,
+__global__ void __launch_bounds__(256) k_train_rows(int n, const uint8_t* __restrict__ px,
                                                     const int32_t* __restrict__ idx, const uint32_t* __restrict__ tmask,
                                                     const uint8_t* __restrict__ eps, float seed_w,
                                                     const uint16_t* __restrict__ wt, const float* __restrict__ w,
@@ -258,6 +264,7 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, int ld, const uint8_t
   const int col_in = lane & 15, rq = (lane >> 4) * 4;  // D layout: rows rq .. rq + 3 of a tile, column col_in
   const int nj3 = wave == 0 ? 5 : 4;                   // output-layer column tiles of this wave
   float* const cp = colpart + (long)blockIdx.x * kBiasCols;
+  uint16_t* const ab = act + (long)blockIdx.x * RT * kActBlk;  // the workgroup's blocks
   WFrags<4, 2> fA;
   WFrags<4, 4> fB0, fB1;
   load_frags(fA, wt + kTrW1T, 64, c0, 16, 4, 0, lane);
@@ -281,21 +288,21 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, int ld, const uint8_t
     sX[r * LX + cc] = f2bf(x);
   }
   __syncthreads();
-  for (int e = tid; e < 64 * (R / 8); e += 256) {  // X feature-major: (feature, 8 rows)
+  for (int e = tid; e < 64 * (R / 8); e += 256) {  // X: (feature, 8 rows)
     const int f = e / (R / 8), rr = (e % (R / 8)) * 8;
     uint16_t h[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) h[j] = sX[(rr + j) * LX + f];
     uint4 v;
     __builtin_memcpy(&v, h, 16);
-    *reinterpret_cast<uint4*>(act + (long)(kActX + f) * ld + r0 + rr) = v;
+    *reinterpret_cast<uint4*>(ab + (rr >> 4) * kActBlk + (kActX + f) * 16 + (rr & 15)) = v;
   }
   {  // layer 1: H1 = relu(X W1 + b1)
     f32x4_t acc[RT][4];
     zero_acc(acc);
     mfma_frags(acc, fA, sX, LX, 0, 4, lane);
     load_frags(fB1, wt + kTrW2T, kNetHid, c0, 16, 4, 128, lane);
-    layer_out<RT>(acc, c0, lane, w + kOffB1, nullptr, sH1, act + (long)kActH1 * ld + r0, ld, nullptr);
+    layer_out<RT>(acc, c0, lane, w + kOffB1, nullptr, sH1, ab + kActH1 * 16, nullptr);
   }
   __syncthreads();
   WFrags<5, 4> fC0, fC1;
@@ -306,7 +313,7 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, int ld, const uint8_t
     load_frags(fC0, wt + kTrW3T, kNetHid, 16 * wave, 64, nj3, 0, lane);
     mfma_frags(acc, fB1, sH1, LH, 128, 4, lane);
     load_frags(fC1, wt + kTrW3T, kNetHid, 16 * wave, 64, nj3, 128, lane);
-    layer_out<RT>(acc, c0, lane, w + kOffB2, nullptr, sH2, act + (long)kActH2 * ld + r0, ld, nullptr);
+    layer_out<RT>(acc, c0, lane, w + kOffB2, nullptr, sH2, ab + kActH2 * 16, nullptr);
   }
   __syncthreads();
   WFrags<4, 4> fD0;
@@ -389,7 +396,7 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, int ld, const uint8_t
   if (lane == 0) s_l[wave] = l;
   __syncthreads();
   if (tid == 0) atomicAdd(loss, (s_l[0] + s_l[1] + s_l[2] + s_l[3]) * inv_n);
-  // db3 column sums (fp32, rows in order); dY feature-major (rows 262..319 zero)
+  // db3 column sums (fp32, rows in order); dY (features 262..319 zero)
   for (int cc = tid; cc < kNetOut; cc += 256) {
     float s = 0.0f;
     for (int r = 0; r < R; ++r) s += sY[r * LY + cc];
@@ -402,7 +409,7 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, int ld, const uint8_t
     for (int j = 0; j < 8; ++j) h[j] = f < 288 ? sDY[(rr + j) * LD + f] : (uint16_t)0;
     uint4 v;
     __builtin_memcpy(&v, h, 16);
-    *reinterpret_cast<uint4*>(act + (long)(kActDY + f) * ld + r0 + rr) = v;
+    *reinterpret_cast<uint4*>(ab + (rr >> 4) * kActBlk + (kActDY + f) * 16 + (rr & 15)) = v;
   }
   WFrags<4, 4> fE0, fE1;
   {  // dH2 = (dY W3^T) * [H2 > 0]
@@ -412,7 +419,7 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, int ld, const uint8_t
     load_frags(fE0, wt + kTrW2R, kNetHid, c0, 16, 4, 0, lane);
     mfma_frags(acc, fD1, sDY, LD, 128, 4, lane);
     load_frags(fE1, wt + kTrW2R, kNetHid, c0, 16, 4, 128, lane);
-    layer_out<RT>(acc, c0, lane, nullptr, sH2, sDH2, act + (long)kActDH2 * ld + r0, ld, cp + kNetHid);
+    layer_out<RT>(acc, c0, lane, nullptr, sH2, sDH2, ab + kActDH2 * 16, cp + kNetHid);
   }
   __syncthreads();
   {  // dH1 = (dH2 W2^T) * [H1 > 0]
@@ -420,7 +427,7 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, int ld, const uint8_t
     zero_acc(acc);
     mfma_frags(acc, fE0, sDH2, LH, 0, 4, lane);
     mfma_frags(acc, fE1, sDH2, LH, 128, 4, lane);
-    layer_out<RT>(acc, c0, lane, nullptr, sH1, nullptr, act + (long)kActDH1 * ld + r0, ld, cp);
+    layer_out<RT>(acc, c0, lane, nullptr, sH1, nullptr, ab + kActDH1 * 16, cp);
   }
 }
 
@@ -429,8 +436,8 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, int ld, const uint8_t
 // rows (a multiple of 32); split s stores its partial products to part + s *
 // kWgPart ([64][256], [256][256], [256][320]; k_grad_reduce adds them in a
 // fixed order).  Wave w owns the 32 x 32 quadrant (w / 2, w % 2) as 2 x 2
-// MFMA tiles; both operands are feature-major rows of act, loaded straight
-// into registers.
+// MFMA tiles; both operands are loaded from act's blocks straight into
+// registers.
 __global__ void __launch_bounds__(256) k_train_wgrad(const uint16_t* __restrict__ act, int ld, int kspan,
                                                      float* __restrict__ part) {
   const int t = blockIdx.x, s = blockIdx.y;
@@ -447,9 +454,10 @@ __global__ void __launch_bounds__(256) k_train_wgrad(const uint16_t* __restrict_
   }
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32, r = lane & 15, kq = (lane >> 4) * 8;
-  const uint16_t* A0 = act + (long)(arow + m0 + wm + r) * ld + kq;
-  const uint16_t* B0 = act + (long)(brow + n0 + wn + r) * ld + kq;
-  const long l16 = 16L * ld;
+  // a step's 32 rows are two blocks: lanes 0 .. 31 read the first, the others the second
+  const uint16_t* A0 = act + (long)(kq >> 4) * kActBlk + (arow + m0 + wm + r) * 16 + (kq & 15);
+  const uint16_t* B0 = act + (long)(kq >> 4) * kActBlk + (brow + n0 + wn + r) * 16 + (kq & 15);
+  constexpr int kF16 = 16 * 16;  // 16 features on
   f32x4_t acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -458,13 +466,14 @@ __global__ void __launch_bounds__(256) k_train_wgrad(const uint16_t* __restrict_
   const int kb = s * kspan, ke = min(ld, kb + kspan);
   int k = kb;
   for (; k + 256 <= ke; k += 256) {  // 8 steps' fragments requested before their MFMAs
+    const uint16_t *Ak = A0 + (long)(k >> 4) * kActBlk, *Bk = B0 + (long)(k >> 4) * kActBlk;
     bf16x8_t a[8][2], b[8][2];
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      a[q][0] = frag(A0 + k + 32 * q);
-      a[q][1] = frag(A0 + l16 + k + 32 * q);
-      b[q][0] = frag(B0 + k + 32 * q);
-      b[q][1] = frag(B0 + l16 + k + 32 * q);
+      a[q][0] = frag(Ak + q * (2 * kActBlk));
+      a[q][1] = frag(Ak + kF16 + q * (2 * kActBlk));
+      b[q][0] = frag(Bk + q * (2 * kActBlk));
+      b[q][1] = frag(Bk + kF16 + q * (2 * kActBlk));
     }
 #pragma unroll
     for (int q = 0; q < 8; ++q)
@@ -475,7 +484,8 @@ __global__ void __launch_bounds__(256) k_train_wgrad(const uint16_t* __restrict_
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[q][i], b[q][j], acc[i][j], 0, 0, 0);
   }
   for (; k < ke; k += 32) {
-    const bf16x8_t a0 = frag(A0 + k), a1 = frag(A0 + l16 + k), b0 = frag(B0 + k), b1 = frag(B0 + l16 + k);
+    const uint16_t *Ak = A0 + (long)(k >> 4) * kActBlk, *Bk = B0 + (long)(k >> 4) * kActBlk;
+    const bf16x8_t a0 = frag(Ak), a1 = frag(Ak + kF16), b0 = frag(Bk), b1 = frag(Bk + kF16);
     acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, acc[0][0], 0, 0, 0);
     acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b1, acc[0][1], 0, 0, 0);
     acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b0, acc[1][0], 0, 0, 0);

@@ -160,8 +160,8 @@ struct NetState {
 };
 
 // Network workspace over `rows` blocks: the inputs of a forward pass (X) and,
-// for training, the batch's feature-major activations and gradients
-// (kActRows x ld bf16, ld = rows rounded up to 32), the k_train_rows
+// for training, the batch's activations and gradients (ld x kActRows bf16,
+// ld = rows rounded up to 32), the k_train_rows
 // workgroups' bias column sums and the weight-gradient partials of up to
 // kMaxSplits batch splits.
 struct NetWork {
@@ -396,7 +396,7 @@ int net_grad_q(mptc_ctx* c, hipStream_t s, NetState& n, NetWork& w, int rows, co
   const int kspan = ((ld + splits - 1) / splits + 31) / 32 * 32;
   const int nwb = (int)grid_for(kNetParams, 256);
   return launch(c, s, KF_NET_FWD, [&] {
-    hipLaunchKernelGGL(k_train_rows<kTrainRT>, dim3(nwg), dim3(256), 0, s, rows, ld, px, idx, target, eps, seed_w, n.wt, n.w,
+    hipLaunchKernelGGL(k_train_rows<kTrainRT>, dim3(nwg), dim3(256), 0, s, rows, px, idx, target, eps, seed_w, n.wt, n.w,
                        n.use_base ? n.base : nullptr, w.act, w.colpart, loss);
     hipLaunchKernelGGL(k_train_wgrad, dim3(kWgTiles, splits), dim3(256), 0, s, w.act, ld, kspan, w.split);
     hipLaunchKernelGGL(k_grad_reduce, dim3(nwb + (kBiasCols + 3) / 4), dim3(256), 0, s, w.split, splits,
