@@ -80,7 +80,11 @@ __global__ void __launch_bounds__(256) k_net_input(const uint8_t* __restrict__ p
 // l % 16, k (l / 16) * 8 .. +7; B column l % 16, k (l / 16) * 8 .. +7; D rows
 // (l / 16) * 4 .. +3, column l % 16.  Every operand fragment is one 16-byte
 // load of 8 consecutive k, so each operand is kept with k contiguous:
-//  - bf16 weight copies (written by the Adam step / k_train_copies; pads stay zero):
+//  - bf16 weight copies (written by the Adam step / k_train_copies; pads stay
+//    zero), [output column][k] in fragment order (wfrag): the 64 lanes' loads
+//    of a fragment are one 1 KB run (as rows they were 16 pieces of 64 bytes,
+//    512 bytes apart, which 256 workgroups take from the same memory channels
+//    at once: k_train_rows 30 us at 4,096 rows, 23 so):
 //      W1T [256][64]  (W1 transposed, k 48..63 zero)      forward, layer 1
 //      W2T [256][256] (W2 transposed)                     forward, layer 2
 //      W3T [272][256] (W3 transposed, rows 262..271 zero)  forward, layer 3
@@ -109,29 +113,33 @@ constexpr int kBiasCols = 2 * kNetHid + kNetOut;           // 774: db1, db2, db3
 constexpr long kWgPart = 64L * 256 + 256L * 256 + 256L * 320;  // floats of one split's weight gradients
 constexpr int kWgTiles = 4 + 16 + 20;                      // 64 x 64 tiles of dW1, dW2, dW3
 
+// position of output column n, input k in a weight copy of ks k-steps of 32
+__device__ __forceinline__ int wfrag(int n, int k, int ks) {
+  return ((((n >> 4) * ks + (k >> 5)) * 4 + ((k >> 3) & 3)) * 16 + (n & 15)) * 8 + (k & 7);
+}
+
 // the bf16 training copies of parameter i (a weight; biases have none)
 __device__ __forceinline__ void store_train_copies(int i, float wi, uint16_t* __restrict__ wt) {
   const uint16_t h = f2bf(wi);
   if (i < kOffB1) {
     const int k = i / kNetHid, n = i % kNetHid;
-    wt[kTrW1T + n * 64 + k] = h;
+    wt[kTrW1T + wfrag(n, k, 2)] = h;
   } else if (i >= kOffW2 && i < kOffB2) {
     const int j = i - kOffW2, k = j / kNetHid, n = j % kNetHid;
-    wt[kTrW2T + n * kNetHid + k] = h;
-    wt[kTrW2R + j] = h;
+    wt[kTrW2T + wfrag(n, k, 8)] = h;
+    wt[kTrW2R + wfrag(k, n, 8)] = h;
   } else if (i >= kOffW3 && i < kOffB3) {
     const int j = i - kOffW3, k = j / kNetOut, n = j % kNetOut;
-    wt[kTrW3T + n * kNetHid + k] = h;
-    wt[kTrW3R + k * 288 + n] = h;
+    wt[kTrW3T + wfrag(n, k, 8)] = h;
+    wt[kTrW3R + wfrag(k, n, 9)] = h;
   }
 }
 
 __device__ __forceinline__ bf16x8_t frag(const uint16_t* p) { return *reinterpret_cast<const bf16x8_t*>(p); }
 
-// The weight fragments of KS k-steps (from k0) of NJ column tiles of a
-// weight copy gB (tile j: output columns col0 + cstep * j .. +15, one row of
-// gB per output column, k contiguous, row stride ldb).  nj (wave-uniform)
-// tiles are loaded.  Loading a chunk before the work that precedes its
+// The weight fragments of KS k-steps (from step k0) of NJ column tiles of a
+// weight copy gB of ksteps k-steps (tile j: output columns 16 (t0 + tstep * j)
+// .. +15).  nj (wave-uniform) tiles are loaded.  Loading a chunk before the work that precedes its
 // MFMAs keeps the L2 round trip off the critical path.
 template <int NJ, int KS>
 struct WFrags {
@@ -139,14 +147,13 @@ struct WFrags {
 };
 
 template <int NJ, int KS>
-__device__ __forceinline__ void load_frags(WFrags<NJ, KS>& f, const uint16_t* __restrict__ gB, int ldb, int col0,
-                                           int cstep, int nj, int k0, int lane) {
-  const int r = lane & 15, kq = (lane >> 4) * 8;
+__device__ __forceinline__ void load_frags(WFrags<NJ, KS>& f, const uint16_t* __restrict__ gB, int ksteps, int t0,
+                                           int tstep, int nj, int k0, int lane) {
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
-      if (j < nj) f.b[ks][j] = frag(gB + (long)(col0 + cstep * j + r) * ldb + k0 + ks * 32 + kq);
+      if (j < nj) f.b[ks][j] = frag(gB + ((t0 + tstep * j) * ksteps + k0 + ks) * 512 + lane * 8);
 }
 
 // acc[i][j] += A x B: A = rows 16 i .. 16 i + 15 of the LDS matrix sA (row
@@ -260,15 +267,15 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, const uint8_t* __rest
   __shared__ uint32_t s_tm[R * 8];
   __shared__ uint8_t s_eps[R * kNetSeeds];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int r0 = blockIdx.x * R, c0 = wave * 64;
+  const int r0 = blockIdx.x * R, c0 = wave * 64, t0 = wave * 4;
   const int col_in = lane & 15, rq = (lane >> 4) * 4;  // D layout: rows rq .. rq + 3 of a tile, column col_in
   const int nj3 = wave == 0 ? 5 : 4;                   // output-layer column tiles of this wave
   float* const cp = colpart + (long)blockIdx.x * kBiasCols;
   uint16_t* const ab = act + (long)blockIdx.x * RT * kActBlk;  // the workgroup's blocks
   WFrags<4, 2> fA;
   WFrags<4, 4> fB0, fB1;
-  load_frags(fA, wt + kTrW1T, 64, c0, 16, 4, 0, lane);
-  load_frags(fB0, wt + kTrW2T, kNetHid, c0, 16, 4, 0, lane);
+  load_frags(fA, wt + kTrW1T, 2, t0, 1, 4, 0, lane);
+  load_frags(fB0, wt + kTrW2T, 8, t0, 1, 4, 0, lane);
   if (tid < R) s_src[tid] = r0 + tid < n ? (idx ? (long)idx[r0 + tid] : (long)(r0 + tid)) : -1;
   __syncthreads();
   // the rows' pixels, target sets and seeds, all requested at once; inputs
@@ -301,7 +308,7 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, const uint8_t* __rest
     f32x4_t acc[RT][4];
     zero_acc(acc);
     mfma_frags(acc, fA, sX, LX, 0, 4, lane);
-    load_frags(fB1, wt + kTrW2T, kNetHid, c0, 16, 4, 128, lane);
+    load_frags(fB1, wt + kTrW2T, 8, t0, 1, 4, 4, lane);
     layer_out<RT>(acc, c0, lane, w + kOffB1, nullptr, sH1, ab + kActH1 * 16, nullptr);
   }
   __syncthreads();
@@ -310,9 +317,9 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, const uint8_t* __rest
     f32x4_t acc[RT][4];
     zero_acc(acc);
     mfma_frags(acc, fB0, sH1, LH, 0, 4, lane);
-    load_frags(fC0, wt + kTrW3T, kNetHid, 16 * wave, 64, nj3, 0, lane);
+    load_frags(fC0, wt + kTrW3T, 8, wave, 4, nj3, 0, lane);
     mfma_frags(acc, fB1, sH1, LH, 128, 4, lane);
-    load_frags(fC1, wt + kTrW3T, kNetHid, 16 * wave, 64, nj3, 128, lane);
+    load_frags(fC1, wt + kTrW3T, 8, wave, 4, nj3, 4, lane);
     layer_out<RT>(acc, c0, lane, w + kOffB2, nullptr, sH2, ab + kActH2 * 16, nullptr);
   }
   __syncthreads();
@@ -322,9 +329,9 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, const uint8_t* __rest
     f32x4_t acc[RT][5];
     zero_acc(acc);
     mfma_frags(acc, fC0, sH2, LH, 0, nj3, lane);
-    load_frags(fD0, wt + kTrW3R, 288, c0, 16, 4, 0, lane);
+    load_frags(fD0, wt + kTrW3R, 9, t0, 1, 4, 0, lane);
     mfma_frags(acc, fC1, sH2, LH, 128, nj3, lane);
-    load_frags(fD1, wt + kTrW3R, 288, c0, 16, 4, 128, lane);
+    load_frags(fD1, wt + kTrW3R, 9, t0, 1, 4, 4, lane);
 #pragma unroll
     for (int j = 0; j < 5; ++j)
       if (j < nj3) {
@@ -416,9 +423,9 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, const uint8_t* __rest
     f32x4_t acc[RT][4];
     zero_acc(acc);
     mfma_frags(acc, fD0, sDY, LD, 0, 4, lane);
-    load_frags(fE0, wt + kTrW2R, kNetHid, c0, 16, 4, 0, lane);
+    load_frags(fE0, wt + kTrW2R, 8, t0, 1, 4, 0, lane);
     mfma_frags(acc, fD1, sDY, LD, 128, 4, lane);
-    load_frags(fE1, wt + kTrW2R, kNetHid, c0, 16, 4, 128, lane);
+    load_frags(fE1, wt + kTrW2R, 8, t0, 1, 4, 4, lane);
     layer_out<RT>(acc, c0, lane, nullptr, sH2, sDH2, ab + kActDH2 * 16, cp + kNetHid);
   }
   __syncthreads();
