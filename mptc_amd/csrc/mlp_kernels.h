@@ -185,21 +185,21 @@ __device__ __forceinline__ void zero_acc(f32x4_t (&acc)[RT][NJ]) {
 }
 
 // Epilogue of a 256-wide layer: wave columns c0 + 16 j + (lane % 16), rows
-// 16 i + (lane / 16) * 4 + t.  H = relu(acc + bias) (forward, mask null) or
+// 16 i + (lane / 16) * 4 + t.  H = relu(acc + bias[j]) (forward, mask null) or
 // acc * [mask > 0] (backward); bf16 to the LDS rows sO (when non-null) and as
 // 4 consecutive rows of one feature to gO (the layer's features in the
 // workgroup's first block);
 // with cpo, the fp32 column sums over the workgroup's rows go to cpo[col].
-template <int RT>
-__device__ __forceinline__ void layer_out(const f32x4_t (&acc)[RT][4], int c0, int lane, const float* __restrict__ bias,
+template <int RT, int NJ>
+__device__ __forceinline__ void layer_out(const f32x4_t (&acc)[RT][NJ], int c0, int lane, const float* bias,
                                           const uint16_t* mask, uint16_t* sO, uint16_t* __restrict__ gO,
                                           float* __restrict__ cpo) {
   constexpr int LH = kNetHid + 8;
   const int col_in = lane & 15, rq = (lane >> 4) * 4;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < NJ; ++j) {
     const int col = c0 + 16 * j + col_in;
-    const float b = bias ? bias[col] : 0.0f;
+    const float b = bias ? bias[j] : 0.0f;
     float cs = 0.0f;
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
@@ -228,27 +228,31 @@ __device__ __forceinline__ void layer_out(const f32x4_t (&acc)[RT][4], int c0, i
   }
 }
 
-// One workgroup (4 waves) per 16 RT batch rows: the forward pass (H1, H2,
+// One workgroup (8 waves) per 16 RT batch rows: the forward pass (H1, H2,
 // logits and seeds), the loss and dY = d(mean loss)/dY, and the backward
 // products dH2 = (dY W3^T) * [H2 > 0], dH1 = (dH2 W2^T) * [H1 > 0], all
 // held in LDS; the weight-gradient operands go out as blocks of act and
 // the bias gradients as this workgroup's column sums of dH1, dH2, dY in fp32
-// (colpart[wg][774]).  Wave w computes columns 64 w .. 64 w + 63 of each
-// 256-wide layer (RT x 4 MFMA tiles) and column tiles w, w + 4, ... of the 17
-// of the output layer.  Batch row r (r < n) takes pair idx[r] (or r); rows
-// n .. ld - 1 are zero in the inputs and gradients.  The weight fragments of
-// each layer are requested in chunks of 4 or 5 k-steps one chunk ahead of
-// their MFMAs, the backward's during the loss.
+// (colpart[wg][774]).  Wave w computes columns 32 w .. 32 w + 31 of each
+// 256-wide layer (RT x 2 MFMA tiles) and column tiles w, w + 8, ... of the 17
+// of the output layer; waves 0 .. 3 take the loss.  A batch of 4,096 rows is
+// one workgroup a CU and a chain of loads and layers, mostly latency: 17.4 us
+// (23.1 with 4 waves, each layer's weights requested in halves a few MFMAs
+// ahead, and the biases after the MFMAs).
+// Batch row r (r < n) takes pair idx[r] (or r); rows n .. ld - 1 are zero in
+// the inputs and gradients.  The weight fragments of a layer are requested a
+// layer ahead of their MFMAs, the last ones before the loss.
 //
 // Loss: -log of the probability the softmax of the 256 logits gives the row's
 // target set (tmask: 8 words, bit L of word L / 32; one bit = the usual
 // cross-entropy), plus seed_w * the mean squared error of the 6 seeds against
 // the endpoints / 255.  d/dy_c of the set term is p_c - [c in set] exp(y_c) /
-// sum_{set} exp(y).  A row with an empty set adds only its seed term.  A wave
-// takes its 4 RT rows at once (64 / (4 RT) lanes per row).  The batch's mean
+// sum_{set} exp(y).  A row with an empty set adds only its seed term.  Each of the
+// four waves takes 4 RT rows at once (64 / (4 RT) lanes per row).  The batch's mean
 // loss is added to *loss (one atomic per workgroup).
+constexpr int kTrainThreads = 512;
 template <int RT>
-__global__ void __launch_bounds__(256) k_train_rows(int n, const uint8_t* __restrict__ px,
+__global__ void __launch_bounds__(kTrainThreads) k_train_rows(int n, const uint8_t* __restrict__ px,
                                                     const int32_t* __restrict__ idx, const uint32_t* __restrict__ tmask,
                                                     const uint8_t* __restrict__ eps, float seed_w,
                                                     const uint16_t* __restrict__ wt, const float* __restrict__ w,
@@ -263,39 +267,58 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, const uint8_t* __rest
   __shared__ __attribute__((aligned(16))) uint16_t sDY[R * LD];   // dY (bf16), columns 262..287 zero
   __shared__ __attribute__((aligned(16))) uint16_t sDH2[R * LH];  // dH2 (bf16)
   __shared__ float s_l[4];
-  __shared__ long s_src[R];
   __shared__ uint32_t s_tm[R * 8];
   __shared__ uint8_t s_eps[R * kNetSeeds];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int r0 = blockIdx.x * R, c0 = wave * 64, t0 = wave * 4;
+  const int r0 = blockIdx.x * R, c0 = wave * 32, t0 = wave * 2;
   const int col_in = lane & 15, rq = (lane >> 4) * 4;  // D layout: rows rq .. rq + 3 of a tile, column col_in
-  const int nj3 = wave == 0 ? 5 : 4;                   // output-layer column tiles of this wave
+  const int nj3 = wave == 0 ? 3 : 2;                   // output-layer column tiles of this wave
   float* const cp = colpart + (long)blockIdx.x * kBiasCols;
   uint16_t* const ab = act + (long)blockIdx.x * RT * kActBlk;  // the workgroup's blocks
-  WFrags<4, 2> fA;
-  WFrags<4, 4> fB0, fB1;
-  load_frags(fA, wt + kTrW1T, 2, t0, 1, 4, 0, lane);
-  load_frags(fB0, wt + kTrW2T, 8, t0, 1, 4, 0, lane);
-  if (tid < R) s_src[tid] = r0 + tid < n ? (idx ? (long)idx[r0 + tid] : (long)(r0 + tid)) : -1;
-  __syncthreads();
-  // the rows' pixels, target sets and seeds, all requested at once; inputs
-  // x = pixel / 255 (pixel-major RGB), columns 48..63 zero
+  // the rows' pixels, target sets and seeds are requested first (pair of row r: -1 past the batch), then the weights
+  auto src_of = [&](int r) -> long { return r0 + r < n ? (idx ? (long)idx[r0 + r] : (long)(r0 + r)) : -1; };
+  constexpr int PX = R * 64 / kTrainThreads;
+  uint8_t pxv[PX];
+#pragma unroll
+  for (int q = 0; q < PX; ++q) {  // input 64 e + lane, e = row (wave-uniform)
+    const long src = src_of(wave + q * (kTrainThreads / 64));
+    pxv[q] = src >= 0 && lane < kNetIn ? px[src * kNetIn + lane] : (uint8_t)0;
+  }
+  uint32_t tmv = 0;
+  uint8_t epv = 0;
   if (tid < R * 8) {
-    const long src = s_src[tid >> 3];
-    s_tm[tid] = src >= 0 ? tmask[src * 8 + (tid & 7)] : 0u;
+    const long src = src_of(tid >> 3);
+    if (src >= 0) tmv = tmask[src * 8 + (tid & 7)];
   }
   if (tid < R * kNetSeeds) {
-    const long src = s_src[tid / kNetSeeds];
-    s_eps[tid] = src >= 0 ? eps[src * kNetSeeds + tid % kNetSeeds] : (uint8_t)0;
+    const long src = src_of(tid / kNetSeeds);
+    if (src >= 0) epv = eps[src * kNetSeeds + tid % kNetSeeds];
   }
-  for (int e = tid; e < R * 64; e += 256) {
-    const int r = e >> 6, cc = e & 63;
-    const long src = s_src[r];
-    const float x = (src >= 0 && cc < kNetIn) ? (float)px[src * kNetIn + cc] * (1.0f / 255.0f) : 0.0f;
-    sX[r * LX + cc] = f2bf(x);
+  WFrags<2, 2> fA;
+  WFrags<2, 4> fB0, fB1;
+  load_frags(fA, wt + kTrW1T, 2, t0, 1, 2, 0, lane);
+  float bias1[2], bias2[2], bias3[3], base3[3];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    bias1[j] = w[kOffB1 + c0 + 16 * j + col_in];
+    bias2[j] = w[kOffB2 + c0 + 16 * j + col_in];
   }
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const int col = 16 * (wave + 8 * j) + col_in;
+    const bool out = j < nj3 && col < kNetOut;
+    bias3[j] = out ? w[kOffB3 + col] : 0.0f;
+    base3[j] = out && base ? base[col] : 0.0f;
+  }
+  load_frags(fB0, wt + kTrW2T, 8, t0, 1, 2, 0, lane);
+  load_frags(fB1, wt + kTrW2T, 8, t0, 1, 2, 4, lane);
+  if (tid < R * 8) s_tm[tid] = tmv;
+  if (tid < R * kNetSeeds) s_eps[tid] = epv;
+#pragma unroll
+  for (int q = 0; q < PX; ++q)  // x = pixel / 255 (pixel-major RGB), columns 48..63 zero
+    sX[(wave + q * (kTrainThreads / 64)) * LX + lane] = f2bf((float)pxv[q] * (1.0f / 255.0f));
   __syncthreads();
-  for (int e = tid; e < 64 * (R / 8); e += 256) {  // X: (feature, 8 rows)
+  for (int e = tid; e < 64 * (R / 8); e += kTrainThreads) {  // X: (feature, 8 rows)
     const int f = e / (R / 8), rr = (e % (R / 8)) * 8;
     uint16_t h[8];
 #pragma unroll
@@ -304,39 +327,41 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, const uint8_t* __rest
     __builtin_memcpy(&v, h, 16);
     *reinterpret_cast<uint4*>(ab + (rr >> 4) * kActBlk + (kActX + f) * 16 + (rr & 15)) = v;
   }
+  WFrags<3, 4> fC0, fC1;
   {  // layer 1: H1 = relu(X W1 + b1)
-    f32x4_t acc[RT][4];
+    f32x4_t acc[RT][2];
     zero_acc(acc);
-    mfma_frags(acc, fA, sX, LX, 0, 4, lane);
-    load_frags(fB1, wt + kTrW2T, 8, t0, 1, 4, 4, lane);
-    layer_out<RT>(acc, c0, lane, w + kOffB1, nullptr, sH1, ab + kActH1 * 16, nullptr);
+    mfma_frags(acc, fA, sX, LX, 0, 2, lane);
+    load_frags(fC0, wt + kTrW3T, 8, wave, 8, nj3, 0, lane);
+    load_frags(fC1, wt + kTrW3T, 8, wave, 8, nj3, 4, lane);
+    layer_out(acc, c0, lane, bias1, nullptr, sH1, ab + kActH1 * 16, nullptr);
   }
   __syncthreads();
-  WFrags<5, 4> fC0, fC1;
+  WFrags<2, 4> fD0;
+  WFrags<2, 5> fD1;
   {  // layer 2: H2 = relu(H1 W2 + b2)
-    f32x4_t acc[RT][4];
+    f32x4_t acc[RT][2];
     zero_acc(acc);
-    mfma_frags(acc, fB0, sH1, LH, 0, 4, lane);
-    load_frags(fC0, wt + kTrW3T, 8, wave, 4, nj3, 0, lane);
-    mfma_frags(acc, fB1, sH1, LH, 128, 4, lane);
-    load_frags(fC1, wt + kTrW3T, 8, wave, 4, nj3, 4, lane);
-    layer_out<RT>(acc, c0, lane, w + kOffB2, nullptr, sH2, ab + kActH2 * 16, nullptr);
+    mfma_frags(acc, fB0, sH1, LH, 0, 2, lane);
+    mfma_frags(acc, fB1, sH1, LH, 128, 2, lane);
+    load_frags(fD0, wt + kTrW3R, 9, t0, 1, 2, 0, lane);
+    load_frags(fD1, wt + kTrW3R, 9, t0, 1, 2, 4, lane);
+    layer_out(acc, c0, lane, bias2, nullptr, sH2, ab + kActH2 * 16, nullptr);
   }
   __syncthreads();
-  WFrags<4, 4> fD0;
-  WFrags<4, 5> fD1;
-  {  // layer 3: Y = H2 W3 + b3 (+ base), column tiles wave, wave + 4, ... of 17
-    f32x4_t acc[RT][5];
+  WFrags<2, 4> fE0, fE1;
+  {  // layer 3: Y = H2 W3 + b3 (+ base), column tiles wave, wave + 8, ... of 17
+    f32x4_t acc[RT][3];
     zero_acc(acc);
     mfma_frags(acc, fC0, sH2, LH, 0, nj3, lane);
-    load_frags(fD0, wt + kTrW3R, 9, t0, 1, 4, 0, lane);
     mfma_frags(acc, fC1, sH2, LH, 128, nj3, lane);
-    load_frags(fD1, wt + kTrW3R, 9, t0, 1, 4, 4, lane);
+    load_frags(fE0, wt + kTrW2R, 8, t0, 1, 2, 0, lane);
+    load_frags(fE1, wt + kTrW2R, 8, t0, 1, 2, 4, lane);
 #pragma unroll
-    for (int j = 0; j < 5; ++j)
+    for (int j = 0; j < 3; ++j)
       if (j < nj3) {
-        const int col = 16 * (wave + 4 * j) + col_in;
-        const float b = col < kNetOut ? w[kOffB3 + col] + (base ? base[col] : 0.0f) : 0.0f;
+        const int col = 16 * (wave + 8 * j) + col_in;
+        const float b = bias3[j] + base3[j];
 #pragma unroll
         for (int i = 0; i < RT; ++i)
 #pragma unroll
@@ -346,7 +371,7 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, const uint8_t* __rest
   __syncthreads();
   const float inv_n = 1.0f / (float)n;
   float l = 0.0f;  // this lane's share of the wave's rows' losses
-  {  // loss and dY: the wave's 4 RT rows at once, LPR lanes per row
+  if (wave < 4) {  // loss and dY: the wave's 4 RT rows at once, LPR lanes per row
     constexpr int LPR = 16 / RT, CPL = kNetLogits / LPR;
     const int r = wave * 4 * RT + lane / LPR, sub = lane % LPR;
     const bool valid = r0 + r < n;
@@ -400,16 +425,16 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, const uint8_t* __rest
     }
   }
   for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
-  if (lane == 0) s_l[wave] = l;
+  if (lane == 0 && wave < 4) s_l[wave] = l;
   __syncthreads();
   if (tid == 0) atomicAdd(loss, (s_l[0] + s_l[1] + s_l[2] + s_l[3]) * inv_n);
   // db3 column sums (fp32, rows in order); dY (features 262..319 zero)
-  for (int cc = tid; cc < kNetOut; cc += 256) {
+  for (int cc = tid; cc < kNetOut; cc += kTrainThreads) {
     float s = 0.0f;
     for (int r = 0; r < R; ++r) s += sY[r * LY + cc];
     cp[2 * kNetHid + cc] = s;
   }
-  for (int e = tid; e < 320 * (R / 8); e += 256) {
+  for (int e = tid; e < 320 * (R / 8); e += kTrainThreads) {
     const int f = e / (R / 8), rr = (e % (R / 8)) * 8;
     uint16_t h[8];
 #pragma unroll
@@ -418,23 +443,20 @@ __global__ void __launch_bounds__(256) k_train_rows(int n, const uint8_t* __rest
     __builtin_memcpy(&v, h, 16);
     *reinterpret_cast<uint4*>(ab + (rr >> 4) * kActBlk + (kActDY + f) * 16 + (rr & 15)) = v;
   }
-  WFrags<4, 4> fE0, fE1;
   {  // dH2 = (dY W3^T) * [H2 > 0]
-    f32x4_t acc[RT][4];
+    f32x4_t acc[RT][2];
     zero_acc(acc);
-    mfma_frags(acc, fD0, sDY, LD, 0, 4, lane);
-    load_frags(fE0, wt + kTrW2R, 8, t0, 1, 4, 0, lane);
-    mfma_frags(acc, fD1, sDY, LD, 128, 4, lane);
-    load_frags(fE1, wt + kTrW2R, 8, t0, 1, 4, 4, lane);
-    layer_out<RT>(acc, c0, lane, nullptr, sH2, sDH2, ab + kActDH2 * 16, cp + kNetHid);
+    mfma_frags(acc, fD0, sDY, LD, 0, 2, lane);
+    mfma_frags(acc, fD1, sDY, LD, 128, 2, lane);
+    layer_out(acc, c0, lane, nullptr, sH2, sDH2, ab + kActDH2 * 16, cp + kNetHid);
   }
   __syncthreads();
   {  // dH1 = (dH2 W2^T) * [H1 > 0]
-    f32x4_t acc[RT][4];
+    f32x4_t acc[RT][2];
     zero_acc(acc);
-    mfma_frags(acc, fE0, sDH2, LH, 0, 4, lane);
-    mfma_frags(acc, fE1, sDH2, LH, 128, 4, lane);
-    layer_out<RT>(acc, c0, lane, nullptr, sH1, nullptr, ab + kActDH1 * 16, cp);
+    mfma_frags(acc, fE0, sDH2, LH, 0, 2, lane);
+    mfma_frags(acc, fE1, sDH2, LH, 128, 2, lane);
+    layer_out(acc, c0, lane, nullptr, sH1, nullptr, ab + kActDH1 * 16, cp);
   }
 }
 

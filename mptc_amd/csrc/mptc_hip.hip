@@ -396,7 +396,7 @@ int net_grad_q(mptc_ctx* c, hipStream_t s, NetState& n, NetWork& w, int rows, co
   const int kspan = ((ld + splits - 1) / splits + 31) / 32 * 32;
   const int nwb = (int)grid_for(kNetParams, 256);
   return launch(c, s, KF_NET_FWD, [&] {
-    hipLaunchKernelGGL(k_train_rows<kTrainRT>, dim3(nwg), dim3(256), 0, s, rows, px, idx, target, eps, seed_w, n.wt, n.w,
+    hipLaunchKernelGGL(k_train_rows<kTrainRT>, dim3(nwg), dim3(kTrainThreads), 0, s, rows, px, idx, target, eps, seed_w, n.wt, n.w,
                        n.use_base ? n.base : nullptr, w.act, w.colpart, loss);
     hipLaunchKernelGGL(k_train_wgrad, dim3(kWgTiles, splits), dim3(256), 0, s, w.act, ld, kspan, w.split);
     hipLaunchKernelGGL(k_grad_reduce, dim3(nwb + (kBiasCols + 3) / 4), dim3(256), 0, s, w.split, splits,
