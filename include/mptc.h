@@ -179,8 +179,9 @@ int32_t mptc_get_stats(mptc_ctx* ctx, mptc_frame_stats* out);
  * "intra_apply", "intra_reeval", "intra_tile", "intra_wave" (the decisions in
  * dependency order), "commit", "unique";
  * learned search: "net_input", "net_l12", "net_l3" (inference), "propose_inter",
- * "top_intra", "lintra_pass"; "net_forward": training steps (the fused
- * forward/loss/backward, weight-gradient and reduction/Adam launches); pruned search:
+ * "top_intra", "lintra_pass"; "net_forward": mptc_net_forward and training
+ * steps (the fused forward/loss/backward, weight-gradient and reduction/Adam
+ * launches); pruned search:
  * "pruned_inter", "pruned_intra", "fold_intra" (only when the window is split
  * into a number of chunks other than 1, 2 or 4; otherwise the intra search
  * takes those decisions)) since it was enabled

@@ -12,8 +12,7 @@
 //          (row dy = 0 holds only dx < 0: the window is causal)
 //
 // Training kernels: k_train_rows, k_train_wgrad, k_grad_reduce (with the
-// Adam step), k_train_copies, k_collect_masks; k_net_input (the inputs of a
-// forward pass).  Search: k_frame_net_input (the network input of a batch)
+// Adam step), k_train_copies, k_collect_masks.  Search: k_frame_net_input (the network input of a batch)
 // and k_lintra_pass (learned intra fixpoint); the inference kernels and the
 // top-k proposal kernels are in net_infer.h.
 #pragma once
@@ -59,18 +58,6 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   uint32_t u;
   __builtin_memcpy(&u, &b, 4);
   return u;
-}
-
-// Network input: x = pixel / 255 (pixel-major RGB), bf16.  Row r of X takes
-// pixel row idx[r] (or r when idx is null).
-__global__ void __launch_bounds__(256) k_net_input(const uint8_t* __restrict__ px, const int32_t* __restrict__ idx,
-                                                   int n, uint16_t* __restrict__ X) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long)n * kNetIn) return;
-  const long row = i / kNetIn;
-  const int c = (int)(i % kNetIn);
-  const long src = idx ? (long)idx[row] : row;
-  X[i] = f2bf((float)px[src * kNetIn + c] * (1.0f / 255.0f));
 }
 
 // ---------------------------------------------------------------------------

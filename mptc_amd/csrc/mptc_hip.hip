@@ -159,14 +159,13 @@ struct NetState {
   uint16_t* pk = nullptr;  // packed inference image (net_infer.h)
 };
 
-// Network workspace over `rows` blocks: the inputs of a forward pass (X) and,
-// for training, the batch's activations and gradients (ld x kActRows bf16,
-// ld = rows rounded up to 32), the k_train_rows
+// Network workspace over `rows` blocks: the inputs of a learned search's
+// forward passes (X) or, for training, the batch's activations and gradients
+// (ld x kActRows bf16, ld = rows rounded up to 32), the k_train_rows
 // workgroups' bias column sums and the weight-gradient partials of up to
 // kMaxSplits batch splits.
 struct NetWork {
   int rows = 0;
-  bool train = false;
   uint16_t *X = nullptr, *act = nullptr;
   float *colpart = nullptr, *split = nullptr;
   void release() {
@@ -227,7 +226,7 @@ struct mptc_ctx {
   // learned proposals
   int mode = MPTC_SEARCH_EXHAUSTIVE, top_k = 8;
   NetState net[2];
-  NetWork nw;  // training and standalone forward passes
+  NetWork nw;  // training
   NetWork ew;  // the encode step's forward passes (max_total rows)
   int n_cu = 256;             // compute units of the device
   uint4* d_h2p = nullptr;     // layer-2 activations of the step (net_infer.h tiles)
@@ -369,16 +368,15 @@ constexpr int kMaxSplits = 16;  // batch splits of the weight gradients
 constexpr int kTrainRT = 1;     // k_train_rows: 16 x kTrainRT batch rows per workgroup
 
 int work_ensure(NetWork& w, int rows, bool train) {
-  if (w.rows >= rows && (w.train || !train)) return MPTC_OK;
+  if (w.rows >= rows) return MPTC_OK;
   w.release();
   const size_t r = (size_t)rows, ld = (r + 31) / 32 * 32;
   int rc;
-  if ((rc = dalloc(&w.X, r * kNetIn))) return rc;
+  if (!train && (rc = dalloc(&w.X, r * kNetIn))) return rc;
   if (train && ((rc = dalloc(&w.act, ld * kActRows)) || (rc = dalloc(&w.colpart, ld / 16 * kBiasCols)) ||
                 (rc = dalloc(&w.split, (size_t)kMaxSplits * kWgPart))))
     return rc;
   w.rows = rows;
-  w.train = train;
   return MPTC_OK;
 }
 
@@ -401,12 +399,6 @@ int net_grad_q(mptc_ctx* c, hipStream_t s, NetState& n, NetWork& w, int rows, co
     hipLaunchKernelGGL(k_train_wgrad, dim3(kWgTiles, splits), dim3(256), 0, s, w.act, ld, kspan, w.split);
     hipLaunchKernelGGL(k_grad_reduce, dim3(nwb + (kBiasCols + 3) / 4), dim3(256), 0, s, w.split, splits,
                        w.colpart, nwg, nwb, n.g, n.w, n.m, n.v, n.wt, adam);
-  });
-}
-
-int net_input_q(mptc_ctx* c, hipStream_t s, const uint8_t* px, const int32_t* idx, int rows, uint16_t* X) {
-  return launch(c, s, KF_NET_INPUT, [&] {
-    hipLaunchKernelGGL(k_net_input, dim3(grid_for(rows * kNetIn, 256)), dim3(256), 0, s, px, idx, rows, X);
   });
 }
 
@@ -546,10 +538,10 @@ int prune_ensure(mptc_ctx* c) {
   return MPTC_OK;
 }
 
-// Fused inference over w.X -> H2 tiles (d_h2p) -> either Y (row-major) or
-// the top-kk admitted offsets of each block into prop.
-int infer_q(mptc_ctx* c, hipStream_t s, const NetState& n, const uint16_t* X, int rows, uint4* h2p, float* Y,
-            int net, int kk, const uint8_t* need, int16_t* prop) {
+// Inference over X -> H2 tiles (d_h2p) -> the top-kk admitted offsets of each
+// block into prop.
+int infer_q(mptc_ctx* c, hipStream_t s, const NetState& n, const uint16_t* X, int rows, uint4* h2p, int net, int kk,
+            const uint8_t* need, int16_t* prop) {
   const int n_tiles = (rows + 31) / 32;
   const unsigned grid = (unsigned)std::max(1, std::min(c->n_cu, (n_tiles + kInferWaves - 1) / kInferWaves));
   const int S = c->cfg.search_area;
@@ -559,9 +551,9 @@ int infer_q(mptc_ctx* c, hipStream_t s, const NetState& n, const uint16_t* X, in
   });
   if (rc) return rc;
   return launch(c, s, KF_NET_L3, [&] {
-    auto kern = Y ? k_net_l3<4, 9> : kk <= 4 ? k_net_l3<4, 8> : kk <= 8 ? k_net_l3<8, 8> : k_net_l3<16, 8>;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * kInferWaves), 0, s, h2p, rows, n.pk, Y, c->d_fr, c->d_sid, net,
-                       S, kk, need, prop, (!Y && n.use_sim) ? n.sim : nullptr, net == 0 ? c->d_rw : c->d_cw,
+    auto kern = kk <= 4 ? k_net_l3<4> : kk <= 8 ? k_net_l3<8> : k_net_l3<16>;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * kInferWaves), 0, s, h2p, rows, n.pk, c->d_fr, c->d_sid, net,
+                       S, kk, need, prop, n.use_sim ? n.sim : nullptr, net == 0 ? c->d_rw : c->d_cw,
                        c->d_own);
   });
 }
@@ -586,7 +578,7 @@ int proposals_q(mptc_ctx* c, hipStream_t s, int net, const uint8_t* need, int16_
     if (rc) return rc;
     x_done = true;
   }
-  return infer_q(c, s, n, c->ew.X, total, c->d_h2p, nullptr, net, c->top_k, need, prop);
+  return infer_q(c, s, n, c->ew.X, total, c->d_h2p, net, c->top_k, need, prop);
 }
 
 // report: the pass writes its count of changed words for the host (the last
@@ -1342,16 +1334,13 @@ int32_t mptc_net_forward(mptc_ctx* c, int32_t net, const uint8_t* d_px, int32_t 
   if (!d_px || !d_out || n < 1) return fail(MPTC_EINVAL, "bad argument");
   if (!c->net[net].ready) return fail(MPTC_ESTATE, "network parameters not set");
   hipStream_t s = c->stream;
-  uint4* h2p = nullptr;
-  if ((rc = dalloc(&h2p, (size_t)(n + 31) / 32 * (kH2TileBytes / 16)))) return rc;
-  if ((rc = work_ensure(c->nw, n, false)) || (rc = net_input_q(c, s, d_px, nullptr, n, c->nw.X)) ||
-      (rc = infer_q(c, s, c->net[net], c->nw.X, n, h2p, d_out, net, 1, nullptr, nullptr))) {
-    (void)hipStreamSynchronize(s);
-    (void)hipFree(h2p);
-    return rc;
-  }
+  const int n_tiles = (n - 1) / 32 + 1;
+  rc = launch(c, s, KF_NET_FWD, [&] {
+    hipLaunchKernelGGL(k_net_forward, dim3(std::min(c->n_cu, n_tiles)), dim3(64 * kFwdWaves), 0, s, d_px, n,
+                       c->net[net].pk, d_out);
+  });
   const hipError_t e = hipStreamSynchronize(s);
-  (void)hipFree(h2p);
+  if (rc) return rc;
   HIP_TRY(e);
   return MPTC_OK;
 }

@@ -1,11 +1,12 @@
-// Inference kernels of the proposal network (mlp_kernels.h): two fused
-// kernels whose weights stay resident in LDS for the whole launch.
+// Inference kernels of the proposal network (mlp_kernels.h).
 //
-//   k_net_l12   x -> h1 -> h2: layers 1 and 2 in registers, h2 stored to HBM
-//               in the operand order layer 3 reads
-//   k_net_l3    h2 -> y: layer 3, then either the 262 outputs (row-major
-//               fp32) or, fused in the epilogue, each block's top-k window
-//               offsets among those its search admits
+//   k_net_forward  pixels -> y: all three layers, their weights in LDS one
+//                  after the other, the activations in registers; the 262
+//                  outputs row-major in fp32
+//   k_net_l12      x -> h1 -> h2: layers 1 and 2 in registers, h2 stored to
+//                  HBM in the operand order layer 3 reads
+//   k_net_l3       h2 -> each block's top-k window offsets among those its
+//                  search admits: layer 3 with the ranking in its epilogue
 //
 // MFMA v_mfma_f32_32x32x16_bf16 computes D[n][m] = sum_k A[n][k] B[k][m] with
 // A = W^T (32 outputs n x 16 inputs k), B = activations^T (16 k x 32 blocks m).
@@ -76,13 +77,26 @@ __global__ void __launch_bounds__(256) k_pack_infer(const float* __restrict__ w,
 // together; with kSwz = 15 they land on 16 different 16-byte bank groups.
 constexpr int kSwz = 15;
 
-// Copies `rows` rows of `chunks` 16-byte chunks into LDS, chunk c of row r at
-// r * chunks + (c ^ (r & kSwz)) (swizzled; chunks >= 16) or r * chunks + c.
-__device__ __forceinline__ void stage_rows(uint4* __restrict__ dst, const uint4* __restrict__ src, int rows,
-                                           int chunks, bool swz) {
-  for (int e = threadIdx.x; e < rows * chunks; e += blockDim.x) {
-    const int r = e / chunks, c = e % chunks;
-    dst[r * chunks + (swz ? (c ^ (r & kSwz)) : c)] = src[e];
+// Copies kRows rows of kChunks 16-byte chunks into LDS with the workgroup's
+// kThreads threads, chunk c of row r at r * kChunks + (c ^ (r & kSwz))
+// (swizzled; kChunks >= 16) or r * kChunks + c.  kAhead chunks a thread are
+// requested before the first is stored, the last ones clamped rather than
+// skipped: one at a time a thread makes 8 to 18 trips to the L2 (k_net_l12
+// 25.6 us, 23.9 so; k_net_l3 at k = 4 43.6 and 41.2).
+template <int kRows, int kChunks, bool kSwizzle, int kThreads, int kAhead = 8>
+__device__ __forceinline__ void stage_rows(uint4* __restrict__ dst, const uint4* __restrict__ src) {
+  constexpr int n = kRows * kChunks;
+#pragma unroll 1
+  for (int e0 = 0; e0 < n; e0 += kAhead * kThreads) {
+    uint4 v[kAhead];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) v[q] = src[min(e0 + q * kThreads + (int)threadIdx.x, n - 1)];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) {
+      const int e = e0 + q * kThreads + (int)threadIdx.x;
+      const int r = e / kChunks, c = e % kChunks;
+      if (e < n) dst[r * kChunks + (kSwizzle ? (c ^ (r & kSwz)) : c)] = v[q];
+    }
   }
 }
 
@@ -122,6 +136,41 @@ __device__ __forceinline__ f32x16_t bias_tile(const float* __restrict__ sb, int 
 constexpr int kInferWaves = 8;  // waves per workgroup of k_net_l3 (255 VGPRs: two per SIMD)
 constexpr int kL12Waves = 16;   // waves per workgroup of k_net_l12 (<= 128 VGPRs: four per SIMD)
 
+// Layer 1 of a tile of 32 blocks, from the lane's inputs xb[s] (k = 16 s + 8 h
+// .. +7 of block m): hb holds the B operands of layer 2.
+__device__ __forceinline__ void net_layer1(const bf16x8_t (&xb)[3], const uint4* sW1, const float* sb, int m, int h,
+                                           bf16x8_t (&hb)[16]) {
+#pragma unroll
+  for (int nb = 0; nb < 8; ++nb) {
+    f32x16_t acc = bias_tile(sb, nb, h);
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      const bf16x8_t a = as_bf16x8(sW1[(nb * 32 + m) * 6 + 2 * s + h]);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, xb[s], acc, 0, 0, 0);
+    }
+    hb[2 * nb] = as_bf16x8(relu_pack(acc, 0));
+    hb[2 * nb + 1] = as_bf16x8(relu_pack(acc, 1));
+    __builtin_amdgcn_sched_barrier(0);  // one accumulator live at a time
+  }
+}
+
+// Output tile nb of layer 2 (before ReLU) from layer 1's hb; at most kAhead
+// weight operands in flight (0: any number).
+template <int kAhead>
+__device__ __forceinline__ f32x16_t net_layer2(const bf16x8_t (&hb)[16], const uint4* sW2, const float* sb, int nb,
+                                               int m, int h) {
+  f32x16_t acc = bias_tile(sb, nb, h);
+  int r = nb * 32 + m;
+  if (kAhead) asm volatile("" : "+v"(r));  // the tile's LDS addresses are computed here, not held in registers from before
+#pragma unroll
+  for (int s = 0; s < 16; ++s) {
+    const bf16x8_t a = as_bf16x8(sW2[r * 32 + ((2 * s + h) ^ (r & kSwz))]);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, hb[s], acc, 0, 0, 0);
+    if (kAhead && s % kAhead == kAhead - 1) __builtin_amdgcn_sched_barrier(0);
+  }
+  return acc;
+}
+
 // Layers 1 and 2.  X: rows x 48 bf16; H2p: per 32-block tile, per k-step s,
 // per lane, the 8 bf16 layer-3 operand values (kH2TileBytes per tile).
 // One workgroup per CU; each wave loops over tiles.
@@ -130,8 +179,8 @@ __global__ void __launch_bounds__(64 * kL12Waves) k_net_l12(const uint16_t* __re
   __shared__ uint4 sW1[kNetHid * kNetIn / 8];   // 24 KiB, rows of 6 chunks
   __shared__ uint4 sW2[kNetHid * kNetHid / 8];  // 128 KiB, rows of 32 chunks, swizzled
   __shared__ __attribute__((aligned(16))) float sb[2 * kNetHid];
-  stage_rows(sW1, reinterpret_cast<const uint4*>(pk + kPkW1), kNetHid, kNetIn / 8, false);
-  stage_rows(sW2, reinterpret_cast<const uint4*>(pk + kPkW2), kNetHid, kNetHid / 8, true);
+  stage_rows<kNetHid, kNetIn / 8, false, 64 * kL12Waves>(sW1, reinterpret_cast<const uint4*>(pk + kPkW1));
+  stage_rows<kNetHid, kNetHid / 8, true, 64 * kL12Waves>(sW2, reinterpret_cast<const uint4*>(pk + kPkW2));
   const float* bias = reinterpret_cast<const float*>(pk + kPkBias);
   for (int i = threadIdx.x; i < 2 * kNetHid; i += blockDim.x) sb[i] = bias[i];
   __syncthreads();
@@ -140,7 +189,7 @@ __global__ void __launch_bounds__(64 * kL12Waves) k_net_l12(const uint16_t* __re
   const int wave_g = blockIdx.x * kL12Waves + (threadIdx.x >> 6);
   for (int tile = wave_g; tile < n_tiles; tile += gridDim.x * kL12Waves) {
     const int row = tile * 32 + m;
-    // layer 1: B operands straight from X (k = 16s + 8h .. +7)
+    // layer 1: B operands straight from X
     bf16x8_t xb[3];
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
@@ -149,31 +198,124 @@ __global__ void __launch_bounds__(64 * kL12Waves) k_net_l12(const uint16_t* __re
       xb[s] = as_bf16x8(v);
     }
     bf16x8_t hb[16];
-#pragma unroll
-    for (int nb = 0; nb < 8; ++nb) {
-      f32x16_t acc = bias_tile(sb, nb, h);
-#pragma unroll
-      for (int s = 0; s < 3; ++s) {
-        const bf16x8_t a = as_bf16x8(sW1[(nb * 32 + m) * 6 + 2 * s + h]);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, xb[s], acc, 0, 0, 0);
-      }
-      hb[2 * nb] = as_bf16x8(relu_pack(acc, 0));
-      hb[2 * nb + 1] = as_bf16x8(relu_pack(acc, 1));
-      __builtin_amdgcn_sched_barrier(0);  // one accumulator live at a time
-    }
+    net_layer1(xb, sW1, sb, m, h, hb);
     // layer 2 (one output tile at a time keeps the live registers to h1 + one accumulator)
     uint4* out = H2p + (size_t)tile * (kH2TileBytes / 16);
 #pragma unroll 1
     for (int nb = 0; nb < 8; ++nb) {
-      f32x16_t acc = bias_tile(sb + kNetHid, nb, h);
-      const int r = nb * 32 + m;
-#pragma unroll
-      for (int s = 0; s < 16; ++s) {
-        const bf16x8_t a = as_bf16x8(sW2[r * 32 + ((2 * s + h) ^ (r & kSwz))]);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, hb[s], acc, 0, 0, 0);
-      }
+      const f32x16_t acc = net_layer2<0>(hb, sW2, sb + kNetHid, nb, m, h);
       out[(2 * nb) * 64 + lane] = relu_pack(acc, 0);
       out[(2 * nb + 1) * 64 + lane] = relu_pack(acc, 1);
+    }
+  }
+}
+
+constexpr int kFwdCols = 3;   // column tiles of 32 outputs taken together
+constexpr int kFwdWaves = 8;  // waves per workgroup of k_net_forward (two per SIMD), two tiles each
+
+// The network's outputs of `rows` rows of 48 pixel bytes (x = byte / 255),
+// Y row-major.  A workgroup takes 16 tiles of 32 rows at a time, two a wave:
+// it stages W1 and W2 in LDS, takes both tiles through layers 1 and 2 into
+// registers, stages W3 over them and finishes both tiles, each W3 operand read
+// once for the two.  Layer 3 multiplies with the operands exchanged (D column =
+// output, rows = blocks), so that a store writes 32 consecutive outputs of two
+// rows, and takes three column tiles at a time, so that a row's stores of 384
+// bytes meet in the L2 (one at a time: 9 us more).  129,600 rows, 136 MB of
+// outputs (21 us at the rate of a large fill): 55 us; as input conversion,
+// layers 1-2 and layer 3 through HBM it was 12 + 26 + 55.
+__global__ void __launch_bounds__(64 * kFwdWaves) k_net_forward(const uint8_t* __restrict__ px, int rows,
+                                                                const uint16_t* __restrict__ pk,
+                                                                float* __restrict__ Y) {
+  __shared__ uint4 sW[kNetHid * (kNetIn + kNetHid) / 8];  // W1 (rows of 6 chunks) and W2 (of 32, swizzled); or W3
+  static_assert(sizeof(sW) >= kL3Rows * kNetHid * 2, "W3 fits in W1's and W2's place");
+  __shared__ __attribute__((aligned(16))) float sb[2 * kNetHid + kL3Rows];
+  uint4* const sW2 = sW + kNetHid * kNetIn / 8;
+  const float* bias = reinterpret_cast<const float*>(pk + kPkBias);
+  for (int i = threadIdx.x; i < 2 * kNetHid + kL3Rows; i += blockDim.x) sb[i] = bias[i];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, m = lane & 31, h = lane >> 5;
+  const int n_tiles = (rows + 31) / 32;
+  const bool wide = (reinterpret_cast<uintptr_t>(px) & 7) == 0;  // rows of 48 bytes: then every load of 8 is aligned
+  for (int base = blockIdx.x; base < n_tiles; base += gridDim.x * (2 * kFwdWaves)) {  // workgroup-uniform
+    if (base != (int)blockIdx.x) __syncthreads();  // every wave is through with the last tiles' W3
+    stage_rows<kNetHid, kNetIn / 8, false, 64 * kFwdWaves>(sW, reinterpret_cast<const uint4*>(pk + kPkW1));
+    stage_rows<kNetHid, kNetHid / 8, true, 64 * kFwdWaves>(sW2, reinterpret_cast<const uint4*>(pk + kPkW2));
+    __syncthreads();
+    // the workgroups' first tiles come first: few rows use one wave of every CU before a second
+    const int tile0 = base + (int)gridDim.x * wave, tile1 = tile0 + (int)gridDim.x * kFwdWaves;
+    bf16x8_t h2[2][16];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int tile = q ? tile1 : tile0;
+      if (tile >= n_tiles) continue;  // wave-uniform
+      const int row = tile * 32 + m;
+      bf16x8_t xb[3];
+#pragma unroll
+      for (int s = 0; s < 3; ++s) {
+        uint2 v = make_uint2(0u, 0u);
+        if (row < rows) {
+          const uint8_t* p = px + (size_t)row * kNetIn + 16 * s + 8 * h;
+          if (wide) {
+            v = *reinterpret_cast<const uint2*>(p);
+          } else {
+            v.x = p[0] | (uint32_t)p[1] << 8 | (uint32_t)p[2] << 16 | (uint32_t)p[3] << 24;
+            v.y = p[4] | (uint32_t)p[5] << 8 | (uint32_t)p[6] << 16 | (uint32_t)p[7] << 24;
+          }
+        }
+        uint32_t w[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t two = (j < 2 ? v.x : v.y) >> (16 * (j & 1));
+          w[j] = pack_bf16x2((float)(two & 255u) * (1.0f / 255.0f), (float)((two >> 8) & 255u) * (1.0f / 255.0f));
+        }
+        xb[s] = as_bf16x8(make_uint4(w[0], w[1], w[2], w[3]));
+      }
+      bf16x8_t hb[16];
+      net_layer1(xb, sW, sb, m, h, hb);
+#pragma unroll
+      for (int nb = 0; nb < 8; ++nb) {
+        const f32x16_t acc = net_layer2<4>(hb, sW2, sb + kNetHid, nb, m, h);
+        h2[q][2 * nb] = as_bf16x8(relu_pack(acc, 0));
+        h2[q][2 * nb + 1] = as_bf16x8(relu_pack(acc, 1));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __syncthreads();
+    stage_rows<kL3Rows, kNetHid / 8, true, 64 * kFwdWaves, 6>(sW, reinterpret_cast<const uint4*>(pk + kPkW3));
+    __syncthreads();
+    if (tile0 >= n_tiles) continue;
+    // kFwdCols columns' tiles at a time: a row's stores of 384 bytes follow one another and meet in the L2
+#pragma unroll 1
+    for (int nb0 = 0; nb0 < kL3Rows / 32; nb0 += kFwdCols) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int tile = q ? tile1 : tile0;
+        if (tile >= n_tiles) continue;
+        int u = nb0 * 32 + m;  // the lane's first output
+        asm volatile("" : "+v"(u));
+        f32x16_t acc[kFwdCols];
+#pragma unroll
+        for (int c = 0; c < kFwdCols; ++c) {
+          const float b = sb[2 * kNetHid + u + 32 * c];
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[c][i] = b;
+        }
+#pragma unroll
+        for (int s = 0; s < 16; ++s)
+#pragma unroll
+          for (int c = 0; c < kFwdCols; ++c) {
+            const bf16x8_t wv = as_bf16x8(sW[(u + 32 * c) * 32 + ((2 * s + h) ^ (u & kSwz))]);
+            acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h2[q][s], wv, acc[c], 0, 0, 0);
+          }
+        const int r0 = tile * 32 + 4 * h;  // D value i: row r0 + 8 (i / 4) + i % 4
+        float* y = Y + (size_t)r0 * kNetOut + u;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int ri = 8 * (i >> 2) + (i & 3);
+#pragma unroll
+          for (int c = 0; c < kFwdCols; ++c)
+            if (r0 + ri < rows && u + 32 * c < kNetOut) y[ri * kNetOut + 32 * c] = acc[c][i];
+        }
+      }
     }
   }
 }
@@ -290,32 +432,31 @@ __device__ __forceinline__ void key_insert(uint32_t (&t)[K], uint32_t key) {
   for (int i = 0; i < K; ++i) t[i] = n[i];
 }
 
-// Layer 3.  NT = 9: writes the 262 outputs of each row to Y (row-major).
-// With sim (kSimBins scores) the top-k adds, to each admitted offset's logit,
+// Layer 3 with the ranking.  With sim (kSimBins scores) the top-k adds, to each admitted offset's logit,
 // sim[index_diff(own word, candidate word)] (words: the candidates' current
 // index words, own: the blocks' fits).
-// NT = 8 (the 256 logit columns only; the endpoint-seed outputs are not
-// computed): for each block g of the batch (rows = total) that `need`
+// The 256 logit columns only (the endpoint-seed outputs are not computed): for
+// each block g of the batch (rows = total) that `need`
 // admits (need null: every block of an inter frame), the top kk <= K
 // admitted offsets by score go to prop[g * kk + i] (-1 past the last).
-template <int K, int NT>
+template <int K>
 __global__ void __launch_bounds__(64 * kInferWaves) k_net_l3(const uint4* __restrict__ H2p, int rows,
-                                                             const uint16_t* __restrict__ pk, float* __restrict__ Y,
+                                                             const uint16_t* __restrict__ pk,
                                                              const FrameDev* __restrict__ fr,
                                                              const uint8_t* __restrict__ sid, int net, int S, int kk,
                                                              const uint8_t* __restrict__ need,
                                                              int16_t* __restrict__ prop, const float* __restrict__ sim,
                                                              const uint32_t* __restrict__ words,
                                                              const uint64_t* __restrict__ own) {
-  static_assert(NT == 8 || NT == 9, "8 logit tiles, or all 9 output tiles");
-  __shared__ uint4 sW3[NT * 32 * kNetHid / 8];  // 128 or 144 KiB, rows of 32 chunks, swizzled
+  constexpr int NT = kNetLogits / 32;
+  __shared__ uint4 sW3[NT * 32 * kNetHid / 8];  // 128 KiB, rows of 32 chunks, swizzled
   __shared__ __attribute__((aligned(16))) float sb[NT * 32];
   __shared__ float s_sim[kSimBins];
   // per wave: the candidate words of a tile of 32 blocks of one frame row,
   // 16 window rows x (32 + 15) columns (similarity term, search mode only)
   constexpr int kWinCols = 32 + kNetWin - 1;
-  __shared__ uint32_t s_win[NT == 8 ? kInferWaves : 1][NT == 8 ? kNetWin * kWinCols : 1];
-  stage_rows(sW3, reinterpret_cast<const uint4*>(pk + kPkW3), NT * 32, kNetHid / 8, true);
+  __shared__ uint32_t s_win[kInferWaves][kNetWin * kWinCols];
+  stage_rows<NT * 32, kNetHid / 8, true, 64 * kInferWaves>(sW3, reinterpret_cast<const uint4*>(pk + kPkW3));
   const float* bias = reinterpret_cast<const float*>(pk + kPkBias) + 2 * kNetHid;
   for (int i = threadIdx.x; i < NT * 32; i += blockDim.x) sb[i] = bias[i];
   if (threadIdx.x < kSimBins) s_sim[threadIdx.x] = sim ? sim[threadIdx.x] : 0.0f;
@@ -340,18 +481,6 @@ __global__ void __launch_bounds__(64 * kInferWaves) k_net_l3(const uint4* __rest
         acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[nb], 0, 0, 0);
       }
     }
-    if (Y) {  // launched with NT = 9 (a runtime test: the compiler then keeps the top-k path free of spills)
-      if (row < rows) {
-#pragma unroll
-        for (int nb = 0; nb < NT; ++nb)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int u = nb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
-            if (u < kNetOut) Y[(size_t)row * kNetOut + u] = acc[nb][i];
-          }
-      }
-      continue;
-    }
     // fused top-k: each lane inserts its 128 logits' keys into a running top
     // K; lane h = 0 merges the partner lane's (l + 32) list and writes
     bool act = row < rows;
@@ -366,7 +495,7 @@ __global__ void __launch_bounds__(64 * kInferWaves) k_net_l3(const uint4* __rest
       act = need ? need[row] != 0 : !dp->is_intra;
       if (act) admitted_words(win_mask(net, S, fbx, fby, dp->bw, dp->bh), vw);
     }
-    if (NT == 8 && sim) {
+    if (sim) {
       // Index similarity: each offset's score gains sim[number of pixels
       // whose index differs between the own word and the candidate's].  The
       // tile's rows are taken in segments that lie in one row of one frame

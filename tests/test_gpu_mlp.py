@@ -54,6 +54,29 @@ def test_forward_matches_oracle(env, n):
     assert err.mean() <= 1e-3 * np.abs(ref).mean(), err.mean()
 
 
+# a tile's remainder, workgroups with one tile, with both of a wave's, and a second round; rows off 8 bytes
+@pytest.mark.parametrize("n,off", [(31, 0), (32, 4), (33, 1), (8193, 0), (70001, 7), (131105, 0)])
+def test_forward_tiles_and_alignment(env, n, off):
+    hip, lib, enc = env
+    log(f"forward n={n} off={off}")
+    p = mlp.he_params(11)
+    enc.net_set_params(1, p)
+    # rows repeat with a period that divides no tile, so a misplaced tile shows
+    px = np.random.default_rng(n).integers(0, 256, (509, 48), dtype=np.uint8)
+    buf = hip.Buffer(n * 48 + off)
+    buf.upload(np.resize(px, (n, 48)), off)
+    guard = np.full(262 * 32, -7.0, np.float32)
+    d_y = hip.Buffer(n * 262 * 4 + guard.nbytes)
+    d_y.upload(guard, n * 262 * 4)
+    enc.net_forward(1, buf.offset(off), n, d_y)
+    y = d_y.download(np.float32, n * 262).reshape(n, 262)
+    assert np.array_equal(d_y.download(np.float32, guard.size, n * 262 * 4), guard)
+    ref = mlp.forward(p, px)["Y"]
+    err = np.abs(y[:509] - ref[:n])
+    assert err.max() <= 2e-2 * np.abs(ref).max(), err.max()
+    assert np.array_equal(y, np.resize(y[:509], (n, 262)))  # a row's result does not depend on its place
+
+
 def test_forward_layout_detects_transposes(env):
     """Structured weights: each output depends on one known input, so a
     transposed or shifted operand layout gives visibly wrong values."""
