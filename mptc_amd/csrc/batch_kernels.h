@@ -387,6 +387,171 @@ __global__ void __launch_bounds__(256) k_inter(const FrameDev* __restrict__ fr, 
   wg_count(&s_acc, n_cand, st->inter_cands);
 }
 
+// Dynamic LDS of k_inter_words for search area S and tiles of tw x 64 / tw
+// blocks: the words of the tile's window (the union of its blocks' windows)
+// and their ids, the word -> id map, and per id its word, its block and its
+// deltas for the tile's 64 blocks (one more row: absent positions).
+struct WordsDims {
+  int uw, pos, ids, hash_log, o_id, o_head, o_word, o_src, o_e, bytes;
+};
+__host__ __device__ __forceinline__ WordsDims words_dims(int S, int tw) {
+  WordsDims D;
+  D.uw = tw - 1 + 2 * S;
+  D.pos = D.uw * (64 / tw - 1 + 2 * S);
+  // two workgroups fit on a CU, which the registers allow too; and more words
+  // than about 7/8 of a block's candidates would not pay for the look-ups
+  D.ids = S <= 8 ? 4 * S * S * 7 / 8 : 448;
+  D.hash_log = S <= 8 ? 10 : 11;  // more buckets than ids and threads: a full map cannot be met
+  D.o_id = (D.pos * 4 + 15) & ~15;
+  D.o_head = (D.o_id + D.pos * 2 + 15) & ~15;
+  D.o_word = D.o_head + (4 << D.hash_log);
+  D.o_src = D.o_word + D.ids * 4;
+  D.o_e = D.o_src + D.ids * 4;
+  D.bytes = D.o_e + (D.ids + 1) * 128;
+  return D;
+}
+constexpr int kWordsMinS = 8, kWordsMaxS = 16;
+constexpr int kWordsWaves = 8;  // each takes a chunk of the window rows
+constexpr uint32_t kNoWord = 0xFFFFu;
+
+// InterBlockSearch as k_inter, for thresholds >= 0 (the selection then depends
+// on the passing deltas alone, and a row without one leaves a summary as it
+// is).  The previous frame's words repeat: each of a block's 4 S^2 candidates
+// that holds the same word gives the same delta.  A workgroup of 8 waves
+// takes a tile of 64 blocks: it finds the distinct words of the tile's window,
+// its waves evaluate each of them once for the 64 blocks (the word is uniform
+// in a wave: its unpacking and table are scalar work), then each takes
+// 2 S / 8 window rows of every block through the rule, with the deltas
+// looked up.  The evaluations bound it: at S = 8, threshold 8, a tile's 511
+// positions hold 128 words where a block has 256 candidates (S = 16: 297 of
+// 1,446, and 1,024).  Twelve streams, 1.5 million blocks, S = 8, threshold 8:
+// 4.2 ms by candidate, 2.4 so.  Requesting the pixels ahead of the window's
+// words takes registers from the evaluations (3.0 ms).
+// A tile with more than WordsDims::ids words evaluates candidate by candidate.
+__global__ void __launch_bounds__(64 * kWordsWaves) k_inter_words(const FrameDev* __restrict__ fr,
+                                                             const uint8_t* __restrict__ tsid, int tw, int S,
+                                                             const uint64_t* __restrict__ own,
+                                                             const uint32_t* __restrict__ rw,
+                                                             const float4* __restrict__ rtab, uint4* __restrict__ summ,
+                                                             size_t sstride, DevStats* __restrict__ st, int thr) {
+  extern __shared__ __align__(16) unsigned char s_words[];
+  __shared__ uint8_t s_snap[512];
+  __shared__ float2 s_ab[4];
+  __shared__ unsigned long long s_acc;
+  __shared__ int s_n;
+  constexpr int kWaves = kWordsWaves, kThreads = 64 * kWaves;
+  const int tile = xcd_block_id();
+  const FrameDev& d = fr[__builtin_amdgcn_readfirstlane(tsid[tile])];
+  if (d.is_intra) return;  // the whole workgroup
+  const WordsDims D = words_dims(S, tw);
+  uint32_t* const w_at = reinterpret_cast<uint32_t*>(s_words);
+  uint16_t* const id_at = reinterpret_cast<uint16_t*>(s_words + D.o_id);
+  int* const head = reinterpret_cast<int*>(s_words + D.o_head);
+  uint32_t* const id_word = reinterpret_cast<uint32_t*>(s_words + D.o_word);
+  int* const id_src = reinterpret_cast<int*>(s_words + D.o_src);
+  int16_t* const E = reinterpret_cast<int16_t*>(s_words + D.o_e);  // [id][lane]
+  const int bw = d.bw, bh = d.bh, base = d.base, W2 = 2 * S, uw = D.uw;
+  const int lt = tile - d.wtile_base, x0 = lt % d.tiles_x * tw, y0 = lt / d.tiles_x * (64 / tw);
+  const int lane = (int)(threadIdx.x & 63), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int lx = lane & (tw - 1), ly = lane >> __builtin_ctz((unsigned)tw), bx = x0 + lx, by = y0 + ly;
+  const bool act = bx < bw && by < bh;
+  const int g = act ? base + by * bw + bx : 0;
+
+  // the window's words (row p / uw is block row y0 - S + p / uw)
+  for (int p = threadIdx.x; p < D.pos; p += kThreads) {
+    const int r = p / uw, j = y0 - S + r, i = x0 - S + p - r * uw;
+    const bool there = j >= 0 && j < bh && i >= 0 && i < bw;
+    w_at[p] = there ? rw[base + j * bw + i] : 0u;
+    id_at[p] = (uint16_t)(there ? 0u : kNoWord);
+  }
+  for (int i = threadIdx.x; i < 1 << D.hash_log; i += kThreads) head[i] = -1;
+  if (threadIdx.x < 64) E[D.ids * 64 + threadIdx.x] = kNoCand;
+  if (threadIdx.x == 0) s_n = 0;
+  load_lds_tables(s_snap, s_ab);  // ends with a barrier
+  // a word's first position takes its bucket and an id, the others note that position
+  for (int p = threadIdx.x; p < D.pos; p += kThreads) {
+    if (id_at[p] == kNoWord) continue;
+    const uint32_t w = w_at[p];
+    uint32_t b = (w * 0x9E3779B1u) >> (32 - D.hash_log);
+    while (__hip_atomic_load(&s_n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <= D.ids) {
+      int at = -1;
+      __hip_atomic_compare_exchange_strong(&head[b], &at, p, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (at < 0) {
+        const int id = atomicAdd(&s_n, 1);
+        if (id < D.ids) {
+          const int r = p / uw;
+          id_word[id] = w;
+          id_src[id] = base + (y0 - S + r) * bw + x0 - S + p - r * uw;
+        }
+        id_at[p] = (uint16_t)id;
+        break;
+      }
+      if (w_at[at] == w) {
+        id_at[p] = (uint16_t)(0x8000 | at);
+        break;
+      }
+      b = (b + 1) & ((1u << D.hash_log) - 1u);
+    }
+  }
+  __syncthreads();
+  const int n_ids = __builtin_amdgcn_readfirstlane(s_n);
+  BlockEval be;
+  if (act) {
+    BlockPx px;
+    load_block(d.rgb, d.width, bx, by, px);
+    make_block_eval(px, own[g], be);
+  }
+  const int rows = (W2 + kWaves - 1) / kWaves, r0 = wv * rows, r1 = min(W2, r0 + rows);
+  ChunkFold cf;
+  if (n_ids <= D.ids) {
+    for (int p = threadIdx.x; p < D.pos; p += kThreads) {
+      const uint32_t v = id_at[p];
+      if (v & 0x8000u) id_at[p] = v == kNoWord ? (uint16_t)D.ids : id_at[v & 0x7FFFu];
+    }
+    for (int id = wv; id < n_ids; id += kWaves) {
+      const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)id_word[id]);
+      const float4 t4 = rtab[__builtin_amdgcn_readfirstlane(id_src[id])];
+      if (act) {
+        const CandResult res = eval_candidate<false>(be, w, CandTab{t4.x, t4.y, t4.z, t4.w}, s_snap, s_ab);
+        E[id * 64 + lane] = (int16_t)(res.valid ? sat16(res.err) : kNoCand);
+      }
+    }
+    __syncthreads();
+    for (int r = r0; r < r1; ++r) {
+      const uint16_t* ids = id_at + (ly + r) * uw + lx;
+      cf.begin_row();
+      for (int t = 0; t < W2; t += 2) {
+        const int e0 = E[ids[t] * 64 + lane], e1 = E[ids[t + 1] * 64 + lane];
+        if (e0 <= thr) cf.step(e0, r * W2 + t, r);
+        if (e1 <= thr) cf.step(e1, r * W2 + t + 1, r);
+      }
+      cf.end_row(r);
+    }
+  } else if (act) {
+    const int t_lo = max(S - bx, 0), t_hi = min(bw - bx + S, W2);
+    for (int r = r0; r < r1; ++r) {
+      const int j = by - S + r;
+      if (j < 0 || j >= bh) continue;
+      cf.begin_row();
+      for (int t = t_lo; t < t_hi; ++t) {
+        const int q = base + j * bw + (bx - S + t);
+        const float4 t4 = rtab[q];
+        const CandResult res = eval_candidate<false>(be, rw[q], CandTab{t4.x, t4.y, t4.z, t4.w}, s_snap, s_ab);
+        cf.step(res.valid ? (int)sat16(res.err) : (int)kNoCand, r * W2 + t, r);
+      }
+      cf.end_row(r);
+    }
+  }
+  unsigned long long n_cand = 0;  // the chunk's window positions inside the frame
+  if (act) {
+    summ[(size_t)wv * sstride + g] = cf.pack();
+    const int lo = max(r0, S - by), hi = min(r1, bh - by + S);
+    if (hi > lo) n_cand = (unsigned long long)(hi - lo) * (min(bw, bx + S) - max(0, bx - S));
+  }
+  wg_count(&s_acc, n_cand, st->inter_cands);
+}
+
 // The inter decision of block g of an inter frame from its chunk summaries
 // (selected position and returned delta) and the previous frame's words rw.
 __device__ __forceinline__ uint64_t inter_decision(const FrameDev& d, int g, int n_chunks, int S, int thr,
