@@ -39,10 +39,10 @@ WORKLOAD = "c2_t0"
 # no FMA), ~28 solve, ~96 quantise + snap, ~24 palette, ~10 validity, ~154
 # integer SSE.
 W_CAND = 600
-# Work of one candidate bound of the pruned search: 36 v_dot4 group sums, 9
-# subtractions for the last group, 20 integer multiply/adds for |S_g|^2, 11
-# fp32 convert/multiply/adds for sum |S_g|^2 / n_g, subtract and compare.
-W_BOUND = 78
+# Work of one candidate bound of the pruned search: per channel 4 v_dot4 for
+# the weighted sum, its conversion, the other sum by subtraction and 5 fp32
+# operations for the quadratic form; then 4 for the limit and the comparison.
+W_BOUND = 37
 # MI355X vector ALU: 157.3 TFLOP/s fp32 = 256 CU x 128 lanes (packed / dual
 # issue) x 2 (FMA) x 2.4 GHz, i.e. 78.6 T lane-ops/s of non-FMA fp32 work.
 VALU_PEAK = 78.6
@@ -164,11 +164,12 @@ def cpu_baseline(spec, steps):
 
 KERNELS = ("fit", "inter", "intra_prep", "intra_dense", "intra_combine", "intra_apply",
            "intra_reeval", "intra_tile", "commit", "unique", "net_input", "net_l12", "net_l3",
-           "propose_inter", "top_intra", "lintra_pass", "pruned_inter", "pruned_intra", "fold_intra")
+           "propose_inter", "top_intra", "lintra_pass", "pruned_inter", "pruned_intra", "fold_intra", "intra_wave")
 
 
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "encode_1080p_plain_hbm_traffic.md")
 KERNEL_SYMBOL = {"inter": "k_inter", "intra_dense": "k_intra_dense", "intra_reeval": "k_intra_reeval",
+                 "intra_wave": "k_intra_wave",
                  "pruned_inter": "k_pruned_search<false>", "pruned_intra": "k_pruned_search<true>"}
 
 
@@ -545,9 +546,10 @@ def measure_config3(hip, lib, steps, warmup):
     enc = lib.Encoder(W, H, spec0["S"], spec0["thr"])
     R = Runner(hip, lib, enc, spec0, frames, max(steps, warmup, 2))
     out = {}
-    # intra fixpoint passes per threshold, the faster of itile_w 0/8/16/32/64
-    # measured on MI355X at this size: tile-resolved 64 x 1 passes at
-    # threshold 8, plain re-fold passes elsewhere
+    # itile_w per threshold, the faster of 0/8/16/32/64 measured on MI355X at
+    # this size: at threshold 8 the windows hold more distinct words than the
+    # decisions in dependency order have room for, and tile-resolved 64 x 1
+    # passes beat re-fold passes
     itile = {8: 64}
     for name in names:
         spec = SEQUENCES[name]

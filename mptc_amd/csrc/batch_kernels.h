@@ -7,16 +7,20 @@
 //                  k_block_prep (mlp_kernels.h) does it together with the
 //                  candidate tables of the reference frames' index words
 //   k_inter        InterBlockSearch + accept test (lane per block, wave tile)
+//   k_inter_words  the same, each distinct word of a tile's window once
 //   k_intra_prep   which blocks need the intra search; initial current words
 //                  (pruned search: their bound tables, empty passing sets)
 //   k_intra_dense  every intra candidate of every such block: stores the error
 //                  deltas E, folds the selection, lists the words that change
+//                  (list form: over k_need_list's searching blocks)
 //   k_intra_apply  the listed words become current (first pass only)
 //   fixpoint passes, each proportional to the work left:
 //     k_intra_reeval    (block, position) pairs that see a changed word
 //     k_intra_select    re-folds those blocks; changed words become current
 //     or k_intra_tile_pass, which also settles the reuse chains inside each
 //                       64-block tile (tuning itile_w)
+//   or, for intra frames at higher thresholds and instead of everything from
+//   k_intra_dense on, k_intra_wave (wave_kernels.h): blocks in dependency order
 //   The intra words are the unique fixpoint of a raster-triangular system
 //   (each block's window holds only earlier blocks); that fixpoint is the
 //   reference's sequential raster-order result.  Passes stop when no word
