@@ -57,8 +57,9 @@ typedef struct {
   int32_t pass_batch; /* intra fixpoint passes queued per convergence check, 1..16 */
   int32_t use_graph;  /* replay the step as captured HIP graphs */
   int32_t win_chunks; /* window tile: the 2S window rows of a block are split into
-                         this many runs scanned by separate waves, 1..8 (above
-                         threshold 4 the inter search of S = 8..16 takes 8) */
+                         this many runs scanned by separate waves, 1..8 (4 or
+                         more is taken as 8 in small batches, and above threshold
+                         4 the inter search of S = 8..16 takes 8) */
   int32_t prune;      /* 1: for thresholds 0..4, evaluate exactly only the candidates an
                          error lower bound cannot rule out (same output);
                          0: evaluate every candidate */

@@ -543,10 +543,22 @@ bool use_words(const mptc_ctx* c) {
 }
 static_assert(kMaxChunks >= kWordsWaves, "a summary for each wave of k_inter_words");
 
-// Chunk summaries the exhaustive inter search leaves per block.
-int inter_chunks(const mptc_ctx* c) {
-  return use_words(c) ? kWordsWaves : chunks_for(c->cfg.search_area, c->tune.win_chunks);
+// Window-row chunks of this batch's searches.  A count of 4 or more becomes 8
+// while that leaves few waves for the work of each: a chunk's wave is a serial
+// chain that a batch of few tiles cannot hide.  The line is 16 waves a CU (what
+// the searches' registers allow at once) at S = 8 and grows with the window.
+// Inter frames, threshold 0, us with 4 / 8 chunks: S = 8 64x64 158 / 136,
+// 640x360 222 / 198, 960x540 359 / 329, 1280x720 288 / 292, 1920x1080 404 / 427;
+// S = 16 256x256 351 / 247, 1920x1080 1,683 / 1,614; S = 32 512x512 1,199 / 816,
+// 1280x720 1,935 / 1,750; S = 7 (2 / 7 chunks) 100x100 271 / 135.
+int window_chunks(const mptc_ctx* c) {
+  const int S = c->cfg.search_area, want = c->tune.win_chunks;
+  const long room = 16L * c->n_cu * std::max(1, S * S / 64);
+  return chunks_for(S, want >= 4 && 8L * c->n_wtiles <= room ? 8 : want);
 }
+
+// Chunk summaries the exhaustive inter search leaves per block.
+int inter_chunks(const mptc_ctx* c) { return use_words(c) ? kWordsWaves : window_chunks(c); }
 
 int prune_ensure(mptc_ctx* c) {
   if (c->d_rbt) return MPTC_OK;
@@ -679,7 +691,7 @@ int queue_prefix(mptc_ctx* c, hipStream_t s, bool fit, bool wave) {
                             c->n_tiles, prune ? c->d_rbt : nullptr);
        })))
     return rc;
-  const int K = chunks_for(S, c->tune.win_chunks);
+  const int K = window_chunks(c);
   // the exhaustive inter searches leave chunk summaries, from which
   // k_intra_prep takes the inter decisions
   const uint4* inter_summ = nullptr;
