@@ -525,9 +525,20 @@ int prepare_batch(mptc_ctx* c, hipStream_t s, int n, const FrameIn* in) {
 // streams, threshold 8: 5.5 ms so, 4.4 with every candidate evaluated.
 constexpr int kPruneMaxThr = 4;
 
+//
+// In a batch of intra frames alone the fixpoint passes, which keep the passing
+// sets up to date, grow with the threshold while the bound's share shrinks; the
+// search is pruned up to threshold 2, above S = 16 up to 1.  Intra frames, ms
+// pruned / not: 1080p S = 8 threshold 0 0.48 / 0.60, 2 1.16 / 1.20, 3 2.11 / 2.11;
+// 768x700 S = 16 0 0.94 / 1.05, 2 2.62 / 2.53, 3 4.92 / 4.17, 4 8.4 / 6.8, S = 8
+// 4 2.2 / 2.0; 1204x668 S = 32 2 23.4 / 20.1, 4 77 / 54.
+int prune_max_thr(const mptc_ctx* c) {
+  return c->any_inter ? kPruneMaxThr : c->cfg.search_area <= 16 ? 2 : 1;
+}
+
 bool use_prune(const mptc_ctx* c) {
   return c->tune.prune && c->mode == MPTC_SEARCH_EXHAUSTIVE && !c->record && c->cfg.err_threshold >= 0 &&
-         c->cfg.err_threshold <= kPruneMaxThr && c->total <= 1 << 27;  // 32-bit offsets of the words' tables
+         c->cfg.err_threshold <= prune_max_thr(c) && c->total <= 1 << 27;  // 32-bit offsets of the words' tables
 }
 
 // The inter search by distinct words (k_inter_words): plain searches above the
