@@ -57,19 +57,16 @@
 #include <stdint.h>
 
 #include "batch_kernels.h"
+#include "wave_ids.h"
 
 namespace mptc {
 
 constexpr int kWaveMaxS = 32;           // a lane per window row and per window column
 constexpr int kWaveIds = 1152;          // most ids: 150 KB of LDS at S = 32
-constexpr unsigned kNoId = 0xFFFFu;
 constexpr int kWaveSpin = 1 << 22;      // polls (about a microsecond each) before a wait gives up
 constexpr int kWaveRoles = 4;           // the waves above
-constexpr int kWaveEval = 12;           // waves that evaluate
 constexpr int kWaveWaves = kWaveRoles + kWaveEval;
-constexpr int kAboveIds = 60;           // of 64 ids, those of wave 1 (the others: wave 2)
 constexpr int kProdBytes = 16 * 96;     // a block's products: per pixel, index value and channel, (p a, p b)
-constexpr int kQuadIds = 384;           // up to so many ids, four lanes evaluate a word
 constexpr int kRawCols = 16;            // columns of the rows above staged for wave 1
 constexpr int kPxBlocks = 16;           // blocks staged at once for the evaluation
 
@@ -250,7 +247,8 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
   extern __shared__ __align__(16) unsigned char s_mem[];
   __shared__ uint8_t s_snap[512];
   __shared__ float2 s_ab[4];
-  __shared__ int s_ticket, s_nused;
+  __shared__ int s_ticket;
+  __shared__ IdCount s_count;
   __shared__ int s_read[2];        // by step parity: the step whose row sets wave 0 has read
   __shared__ int s_fail[2];        // by step parity: set in a step, read in the next
   __shared__ uint32_t s_blk[4][16];  // block b & 3: its 12 channel words, own word, own error, need
@@ -274,7 +272,7 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
 
   if (threadIdx.x == 0) {
     s_ticket = (int)atomicAdd(&st->wave_ticket, 1u);
-    s_nused = 0;
+    s_count = IdCount{};
     s_fail[0] = s_fail[1] = 0;
     s_read[0] = s_read[1] = -4;
   }
@@ -337,7 +335,7 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
         const uint32_t need = s_blk[p & 3][14];
         const unsigned start_id = gid[p & rmask];
         const unsigned id_out = p >= S ? gid[(p - S) & rmask] : kNoId;  // leaves row 0
-        const int nu = s_nused;
+        const int nu = __builtin_amdgcn_readfirstlane(s_count.before(p));
         unsigned sel_id = start_id;
         bool bad = false;
         if (__builtin_amdgcn_readfirstlane((int)need) != 0) {
@@ -427,6 +425,7 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
     uint64_t v = 0;
     float4 t0 = make_float4(0.f, 0.f, 0.f, 0.f);
     bool t_ok = false, dead = false;
+    int n_ids = 0;  // one more than the highest id given out
     // more: the entry for r + 1 has been fetched too
     auto insert = [&](int r, bool more) -> bool {
       const int p = r - 1;
@@ -454,7 +453,7 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
         lds_order();
         const bool first_live = fresh && id != kNoId && lastany[id] >= p - S;  // another word's, still in use
         const int n = (int)__popcll(fm), rank = (int)__popcll(fm & ((1ull << lane) - 1));
-        int got = 0, used = 0;
+        int got = 0;
         for (int chunk = 0; got < n; chunk += 64) {  // the lowest ids that no column holds
           if (chunk >= D.ids) return false;
           unsigned long long fb = __ballot(lane < kAboveIds && lastany[chunk + lane] < p - S);
@@ -462,11 +461,10 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
             const int b = __builtin_ctzll(fb);
             fb &= fb - 1;
             if (fresh && rank == got) id = (unsigned)(chunk + b);
-            used = chunk + b + 1;
+            n_ids = max(n_ids, chunk + b + 1);
             ++got;
           }
         }
-        if (lane == 0) atomicMax(&s_nused, used);
         const unsigned mine = id;
         if (fresh) {
           if (first_live) h = h2;
@@ -486,6 +484,7 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
         }
       }
       if (has) gid[lane * D.ring + (col & rmask)] = (uint16_t)id;
+      if (lane == 0) s_count.publish(p, 0, n_ids);
       v = raw[(lane < W2 ? lane : 0) * kRawCols + ((r + 1) & (kRawCols - 1))];
       t_ok = more && (lane == 0 ? r + 1 >= 0 : act && fin_is(v)) && col + 1 < bw;
       if (t_ok) t0 = ctab[fin_root(v)];
@@ -532,7 +531,7 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
     // pv: that row from column pb, nB of them final; pn: the poll in flight,
     // taken three steps after it was issued or when it is needed.  Its own ids:
     // those with (id & 63) >= kAboveIds.
-    int cB = y < 1 ? bw : 0, pb = 0, nB = 0, pn_at = -1, pn_step = 0;
+    int cB = y < 1 ? bw : 0, pb = 0, nB = 0, pn_at = -1, pn_step = 0, n_ids = 0;
     uint64_t pv = 0, pn = 0;
     bool dead = false;
     auto insert = [&](int p) -> bool {
@@ -574,11 +573,11 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
             }
             if (nid < 0) return false;
             id = (unsigned)nid;
+            n_ids = max(n_ids, nid + 1);
             if (lane == 0) {
               wr[id] = (uint64_t)rt << 32 | w;
               head[h] = (uint16_t)id;
               tab[id] = ctab[rt];
-              atomicMax(&s_nused, nid + 1);
             }
           }
           if (lane == 0) {
@@ -593,7 +592,10 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
           pn_step = p;
           pn = cB + lane < bw ? fin_load(fin + row0 - bw + cB + lane) : 0;
         }
-        if (cB > req) return true;
+        if (cB > req) {
+          if (lane == 0) s_count.publish(p, 1, n_ids);
+          return true;
+        }
         if (!gb) {
           if (give_up(spin)) return false;
         }
@@ -729,8 +731,9 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
       if (b < bw && __builtin_amdgcn_readfirstlane((int)s_blk[b & 3][14]) != 0) {
         int16_t* En = E + (b & 1) * D.ids;
         const uint32_t* blk = s_blk[b & 3];
-        const int nu = s_nused;
-        if (nu <= kQuadIds) {
+        const int nu = __builtin_amdgcn_readfirstlane(s_count.before(p));
+        const EvalSplit sp = eval_split(nu, ev, lane);
+        if (sp.quad) {
           ce.sq = 0;
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
@@ -739,7 +742,7 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
           }
           ce.own = blk[12];
           ce.orig = (int)blk[13];
-          for (int i = ev * 16 + (lane >> 2); i < nu; i += kWaveEval * 16) {
+          for (int i = sp.first; i < nu; i += sp.stride) {
             int e = kNoCand;
             if (lastany[i] >= p - S)
               e = eval_candidate_quad(ce, (uint32_t)wr[i], tab[i], s_snap, prod + (b & 1) * kProdBytes);
@@ -755,7 +758,7 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
           }
           be.own = blk[12];
           be.orig = (int)blk[13];
-          for (int i = ev * 64 + lane; i < nu; i += kWaveEval * 64) {
+          for (int i = sp.first; i < nu; i += sp.stride) {
             int16_t e = kNoCand;
             if (lastany[i] >= p - S) {
               const float4 t4 = tab[i];

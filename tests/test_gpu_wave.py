@@ -113,3 +113,18 @@ def test_intra_wave_matches_tile_passes(w, h, S, thr, seed):
     for i, r in enumerate(runs):
         compare_results(r, want, f"{w}x{h} S={S} thr={thr} run {i}")
         assert np.array_equal(r["kind"], want["kind"])
+
+
+@pytest.mark.parametrize("S,thr", [(9, 300), (10, 8), (12, 300), (16, 8), (16, 300)])
+def test_rows_that_pass_the_four_lane_limit(enc, orc, S, thr):
+    """Rows that begin with few distinct words and end with more than four lanes
+    each are kept for: the split of the ids changes in the middle of them."""
+    w, h = 320, 128
+    rgb = _frame("flat", w, h, 3)
+    noise = _frame("noise", w, h, 4)
+    for i, x0 in enumerate(range(0, w, 32)):  # block rows pass the limit at different columns
+        y0 = (40 + 24 * i) % h
+        rgb[y0:, x0 + 16:x0 + 32] = noise[y0:, x0 + 16:x0 + 32]
+    rgb[:, w // 2:] = noise[:, w // 2:]
+    log(f"S={S} thr={thr}")
+    _intra(enc, orc, rgb, S, thr)
