@@ -27,6 +27,36 @@ struct IdCount {
   }
 };
 
+// Waves 1 and 2 look words up in one map while each may give an id of its own
+// that no column holds to another word.  Each reads and writes the ids' words
+// and the last columns they were seen at through a T: last, word, set_word,
+// set_table, raise, and order, which keeps the wave's accesses on either side
+// of it in that order.
+//
+// Whether id i (kNoId: none) is word w's.  Another wave's id has to be in use
+// (seen at column `oldest` or later: then its word does not change in this
+// step), and the column is read before the word: an id that its owner puts to
+// use meanwhile has its new word by the time the new column shows.  The other
+// way round, the old word with the new column passes for an id in use.
+template <typename T>
+__host__ __device__ __forceinline__ bool id_holds(const T& t, unsigned i, uint32_t w, bool own, int oldest) {
+  const unsigned at = i != kNoId ? i : 0u;
+  const int last = t.last(at);
+  t.order();
+  const uint32_t word = t.word(at);
+  return i != kNoId && word == w && (own || last >= oldest);
+}
+
+// The owner's part, after set_word: the table of id `given`, then the column of
+// `id` (another id of the same word where the wave found one).
+template <typename T, typename Table>
+__host__ __device__ __forceinline__ void id_publish(const T& t, unsigned given, const Table& table, unsigned id,
+                                                    int column) {
+  t.set_table(given, table);
+  t.order();
+  t.raise(id, column);
+}
+
 // The ids (below n_ids) that a lane of evaluating wave ev takes: first, then
 // every stride-th.
 struct EvalSplit {

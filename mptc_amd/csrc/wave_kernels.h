@@ -125,6 +125,19 @@ __device__ __forceinline__ void lds_order() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The id tables in LDS, as wave_ids.h accesses them.
+struct WaveIds {
+  int* lastany;
+  uint64_t* wr;
+  float4* tab;
+  __device__ __forceinline__ int last(unsigned i) const { return lastany[i]; }
+  __device__ __forceinline__ uint32_t word(unsigned i) const { return (uint32_t)wr[i]; }
+  __device__ __forceinline__ void set_word(unsigned i, uint64_t v) const { wr[i] = v; }
+  __device__ __forceinline__ void set_table(unsigned i, const float4& t) const { tab[i] = t; }
+  __device__ __forceinline__ void raise(unsigned i, int column) const { atomicMax(&lastany[i], column); }
+  __device__ __forceinline__ void order() const { lds_order(); }
+};
+
 template <int kCtrl, int kRows>
 __device__ __forceinline__ int dpp_min(int v) {
   return min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, kCtrl, kRows, 0xf, false));
@@ -265,6 +278,7 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
   uint16_t* head = reinterpret_cast<uint16_t*>(s_mem + D.o_head);
   uint16_t* gid = reinterpret_cast<uint16_t*>(s_mem + D.o_gid);
   uint8_t* lastcol = reinterpret_cast<uint8_t*>(s_mem + D.o_lcol);
+  const WaveIds ids{lastany, wr, tab};
 
   const int lane = (int)(threadIdx.x & 63);
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -440,10 +454,7 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
       uint32_t h = wave_hash(w, D.bucket_log);
       const uint32_t h2 = wave_hash2(w, D.bucket_log);
       unsigned id = head[h], id2 = head[h2];
-      // an id of wave 2's that no column holds may get another word at any time
-      auto is = [&](unsigned i) {
-        return i != kNoId && (uint32_t)wr[i] == w && ((i & 63u) < kAboveIds || lastany[i] >= p - S);
-      };
+      auto is = [&](unsigned i) { return id_holds(ids, i, w, (i & 63u) < kAboveIds, p - S); };
       const bool hit1 = has && is(id), hit2 = has && is(id2), hit = hit1 || hit2;
       if (hit2 && !hit1) id = id2;
       if (hit) atomicMax(&lastany[id], seen);
@@ -468,7 +479,7 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
         const unsigned mine = id;
         if (fresh) {
           if (first_live) h = h2;
-          wr[id] = v & 0x7FFFFFFFFFFFFFFFull;
+          ids.set_word(id, v & 0x7FFFFFFFFFFFFFFFull);
           head[h] = (uint16_t)id;
         }
         lds_order();
@@ -479,8 +490,7 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
         if (fresh) {
           // an id given up for an equal word's keeps this word (a bucket may still name it), so its table too
           if (!t_ok) t0 = ctab[fin_root(v)];
-          tab[mine] = t0;
-          atomicMax(&lastany[id], seen);
+          id_publish(ids, mine, t0, id, seen);
         }
       }
       if (has) gid[lane * D.ring + (col & rmask)] = (uint16_t)id;
@@ -551,15 +561,15 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
           const uint32_t rt = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(pv >> 32), cB - pb) & 0x7FFFFFFFu;
           uint32_t h = wave_hash(w, D.bucket_log);
           const uint32_t h2 = wave_hash2(w, D.bucket_log);
-          unsigned id = head[h];
-          const unsigned id2 = head[h2];
-          // an id of wave 1's that no column holds may get another word at any time
+          // the lanes read the same, but not all at once: wave 1 may write in between, so one lane's reads count
+          unsigned id = (unsigned)__builtin_amdgcn_readfirstlane((int)head[h]);
+          const unsigned id2 = (unsigned)__builtin_amdgcn_readfirstlane((int)head[h2]);
           auto is = [&](unsigned i) {
-            return i != kNoId && (uint32_t)wr[i] == w && ((i & 63u) >= kAboveIds || lastany[i] >= p - S);
+            return __builtin_amdgcn_readfirstlane((int)id_holds(ids, i, w, (i & 63u) >= kAboveIds, p - S)) != 0;
           };
           const bool hit1 = is(id), hit2 = is(id2);
           if (hit2 && !hit1) id = id2;
-          if (__ballot(hit1 || hit2) == 0ull) {
+          if (!hit1 && !hit2) {
             if (id != kNoId && lastany[id] >= p - S) h = h2;  // the first bucket's word is still in use
             int nid = -1;
             constexpr int kOwn = 64 - kAboveIds, kAt = 64 / kOwn * 64;  // its ids of 64 / kOwn chunks at a time
@@ -575,15 +585,14 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
             id = (unsigned)nid;
             n_ids = max(n_ids, nid + 1);
             if (lane == 0) {
-              wr[id] = (uint64_t)rt << 32 | w;
+              ids.set_word(id, (uint64_t)rt << 32 | w);
               head[h] = (uint16_t)id;
-              tab[id] = ctab[rt];
+              id_publish(ids, id, ctab[rt], id, cB);
             }
+          } else if (lane == 0) {
+            ids.raise(id, cB);
           }
-          if (lane == 0) {
-            atomicMax(&lastany[id], cB);
-            gid[D.ring + (cB & rmask)] = (uint16_t)id;
-          }
+          if (lane == 0) gid[D.ring + (cB & rmask)] = (uint16_t)id;
           lds_order();
           ++cB;
         }

@@ -14,9 +14,78 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 MOST_IDS = 1152
 
 SOURCE = """
+#include <functional>
+#include <vector>
 #include "wave_ids.h"
 using namespace mptc;
+// one id: the last column it was seen at, its word and its table
+struct Id {
+  int last;
+  uint32_t word;
+  int table;
+};
+// the owner's writes in its order, for the reader to meet at any point
+struct Owner {
+  Id& id;
+  std::vector<std::function<void()>>& ops;
+  void set_word(unsigned, uint64_t v) const { ops.push_back([this, v] { id.word = (uint32_t)v; }); }
+  void set_table(unsigned, int t) const { ops.push_back([this, t] { id.table = t; }); }
+  void raise(unsigned, int c) const { ops.push_back([this, c] { if (c > id.last) id.last = c; }); }
+  void order() const {}
+};
+// a reader before whose k-th read at[k] of the writes are done
+struct Reader {
+  Id& id;
+  std::vector<std::function<void()>>& ops;
+  const int* at;
+  mutable int k, done;
+  void upto(int n) const { while (done < n) ops[done++](); }
+  int last(unsigned) const { upto(at[k++]); return id.last; }
+  uint32_t word(unsigned) const { upto(at[k++]); return id.word; }
+  void order() const {}
+};
+// the test the other way round: the word first
+static bool holds_word_first(const Reader& t, unsigned i, uint32_t w, bool own, int oldest) {
+  return t.word(i) == w && (own || t.last(i) >= oldest);
+}
+static int g_log[8], g_n;
+struct Logged {
+  int last(unsigned) const { g_log[g_n++] = 1; return 0; }
+  uint32_t word(unsigned) const { g_log[g_n++] = 2; return 0; }
+  void set_table(unsigned, int) const { g_log[g_n++] = 3; }
+  void raise(unsigned, int) const { g_log[g_n++] = 4; }
+  void order() const { g_log[g_n++] = 0; }
+};
 extern "C" {
+// Another wave's id, seen at column `last` with word `old`; its owner gives it
+// to word `fresh` at column `now` if no column holds it.  A reader looks for
+// `want` with at[0] and at[1] of the owner's writes done before its two reads.
+// 1: an id in use and right, or none; 0: an id that holds another word (or no table).
+int lookup(int last, unsigned old, unsigned fresh, int now, unsigned want, int oldest, const int* at, int word_first) {
+  Id id{last, old, (int)old};
+  std::vector<std::function<void()>> ops;
+  const Owner o{id, ops};
+  if (last < oldest) {
+    o.set_word(3, fresh);
+    id_publish(o, 3, (int)fresh, 3, now);
+  }
+  const int n = (int)ops.size();
+  const int seq[2] = {at[0] < n ? at[0] : n, at[1] < n ? at[1] : n};
+  const Reader r{id, ops, seq, 0, 0};
+  const bool hit = word_first ? holds_word_first(r, 3, want, false, oldest) : id_holds(r, 3, want, false, oldest);
+  r.upto(n);
+  return !hit || (id.word == want && id.table == (int)want);
+}
+// the accesses of a look-up and of a publication: 0 order, 1 column, 2 word, 3 table, 4 column raised
+int accesses(int publish, int* out) {
+  g_n = 0;
+  if (publish)
+    id_publish(Logged{}, 1, 0, 1, 0);
+  else
+    (void)id_holds(Logged{}, 1, 0, false, 0);
+  for (int i = 0; i < g_n; ++i) out[i] = g_log[i];
+  return g_n;
+}
 static IdCount count;
 int waves() { return kWaveEval; }
 int quad_ids() { return kQuadIds; }
@@ -87,3 +156,33 @@ def test_differing_counts_would_leave_ids_out(ids):
     q = ids.quad_ids()
     h = _hits(ids, [q - 4] * 8 + [q + 61] * 4)
     assert (h[:q - 4] == 0).sum() > 100
+
+
+def _lookups(ids, word_first):
+    """Wrong outcomes over every order of the reader's two accesses and the
+    owner's writes, for ids in use, just out of use and never used."""
+    wrong = runs = 0
+    for last in (-(1 << 30), 4, 5, 6, 30):
+        for fresh in (7, 8):
+            for want in (7, 8):
+                for a in range(4):
+                    for b in range(a, 4):
+                        at = (C.c_int * 2)(a, b)
+                        wrong += not ids.lookup(last, 7, fresh, 30, want, 6, at, word_first)
+                        runs += 1
+    assert runs == 5 * 4 * 10
+    return wrong
+
+
+def test_an_id_found_in_use_holds_the_word(ids):
+    assert _lookups(ids, 0) == 0
+
+
+def test_the_word_before_the_column_is_caught(ids):
+    assert _lookups(ids, 1) > 0
+
+
+def test_accesses_are_ordered(ids):
+    out = (C.c_int * 8)()
+    assert out[:ids.accesses(0, out)] == [1, 0, 2]
+    assert out[:ids.accesses(1, out)] == [3, 0, 4]
