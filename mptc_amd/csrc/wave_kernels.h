@@ -660,8 +660,11 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
         const unsigned id_out = out ? gid[lane * D.ring + ((p - S) & rmask)] : kNoId;
         const bool last = id_out != kNoId && lastcol[id_out * W2 + lane] == (uint8_t)(p - S) && id_out != id_in;
         bad = (in && id_in == kNoId) || (out && id_out == kNoId);
-        while (__hip_atomic_load(&s_read[p & 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != p) {
-        }
+        for (int spin = 0; __hip_atomic_load(&s_read[p & 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != p;)
+          if (++spin > kWaveSpin) {  // wave 0 stores it on every path of its step
+            bad = true;
+            break;
+          }
         lds_order();
         if (id_in != kNoId) enter(id_in, p + S);
         if (last) leave(id_out);

@@ -186,3 +186,14 @@ def test_accesses_are_ordered(ids):
     out = (C.c_int * 8)()
     assert out[:ids.accesses(0, out)] == [1, 0, 2]
     assert out[:ids.accesses(1, out)] == [3, 0, 4]
+
+
+def test_every_wait_counts_its_polls():
+    """The loops of k_intra_wave that wait for another wave or row give up after
+    a number of polls."""
+    import re
+    lines = open(os.path.join(ROOT, "mptc_amd", "csrc", "wave_kernels.h")).read().split("\n")
+    waits = [i for i, t in enumerate(lines) if re.match(r"\s*(while|for) \(.*(atomic_load|fin_is|fin_load)", t)]
+    assert len(waits) == 3
+    for i in waits:
+        assert re.search(r"give_up\(|> kWaveSpin", "\n".join(lines[i:i + 4])), lines[i]
