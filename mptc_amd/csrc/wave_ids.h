@@ -12,6 +12,18 @@ constexpr int kAboveIds = 60;   // of 64 ids, those of wave 1 (the others: wave 
 constexpr int kWaveEval = 12;   // waves that evaluate
 constexpr int kQuadIds = 384;   // up to so many ids, four lanes evaluate a word
 
+// How many ids a window of search area S has: every position of it, and of the
+// columns ahead of it, distinct, in pairs of 64-id chunks; at S = 32 as many as
+// LDS holds.  At least 384, of which wave 2 has 24: the words of the row above
+// alone are up to 2 S + 4 at a time, and one that the other rows repeat keeps
+// its id (with 128 ids at S = 4, 8 of them wave 2's, 1080p frames gave up).
+constexpr int kWaveLook = 2;  // columns of the row above that may enter early
+constexpr int kWaveIds = 1152, kWaveMinIds = 384;
+constexpr __host__ __device__ int wave_id_count(int S) {
+  const int ids = ((2 * S * (2 * S + 4 + kWaveLook) + 8) * 64 / kAboveIds + 127) / 128 * 128;
+  return ids < kWaveMinIds ? kWaveMinIds : ids < kWaveIds ? ids : kWaveIds;
+}
+
 // One more than the highest id in use, by the parity of the step and the wave
 // (0: wave 1, 1: wave 2) that gave it out.  A step's readers take the count
 // that the step before left, which nobody changes meanwhile: the waves that

@@ -62,7 +62,6 @@
 namespace mptc {
 
 constexpr int kWaveMaxS = 32;           // a lane per window row and per window column
-constexpr int kWaveIds = 1152;          // most ids: 150 KB of LDS at S = 32
 constexpr int kWaveSpin = 1 << 22;      // polls (about a microsecond each) before a wait gives up
 constexpr int kWaveRoles = 4;           // the waves above
 constexpr int kWaveWaves = kWaveRoles + kWaveEval;
@@ -88,10 +87,8 @@ constexpr __host__ __device__ WaveDims wave_dims(int S) {
   while (d.ring < 2 * S + 8) d.ring *= 2;
   // columns of the row above that may enter early: a column's ring slot is
   // written only after the column a ring before it left the window
-  d.look = 2;
-  // every position of the window and of the columns ahead of it distinct; pairs of 64-id chunks
-  const int ids = ((2 * S * (2 * S + 4 + d.look) + 8) * 64 / kAboveIds + 127) / 128 * 128;
-  d.ids = ids < kWaveIds ? ids : kWaveIds;
+  d.look = kWaveLook;
+  d.ids = wave_id_count(S);
   d.bucket_log = S <= 8 ? 10 : 12;
   int o = 0;
   d.o_tab = wave_take(o, 16 * d.ids);
@@ -108,7 +105,7 @@ constexpr __host__ __device__ WaveDims wave_dims(int S) {
   d.bytes = o;
   return d;
 }
-static_assert(wave_dims(kWaveMaxS).bytes <= 159 * 1024, "the window fits the LDS of a compute unit");
+static_assert(wave_dims(kWaveMaxS).bytes <= 159 * 1024, "the window fits the LDS of a compute unit");  // 150 KB
 
 // Barrier over the workgroup's LDS: outstanding global loads stay in flight.
 __device__ __forceinline__ void lds_barrier() {

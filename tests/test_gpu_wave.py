@@ -128,3 +128,13 @@ def test_rows_that_pass_the_four_lane_limit(enc, orc, S, thr):
     rgb[:, w // 2:] = noise[:, w // 2:]
     log(f"S={S} thr={thr}")
     _intra(enc, orc, rgb, S, thr)
+
+
+@pytest.mark.parametrize("S,thr", [(2, 8), (3, 8), (4, 8), (4, 32), (5, 6), (6, 8)])
+def test_small_windows_have_ids_enough(enc, orc, S, thr):
+    """Rows of many reused words at small search areas are decided without the
+    fixpoint passes."""
+    log(f"S={S} thr={thr}")
+    rgb = _frame("soft", 480, 256, 40 + S)
+    _intra(enc, orc, rgb, S, thr)
+    assert enc.stats()["intra_iterations"] == 1

@@ -89,6 +89,9 @@ int accesses(int publish, int* out) {
 static IdCount count;
 int waves() { return kWaveEval; }
 int quad_ids() { return kQuadIds; }
+int id_count(int S) { return wave_id_count(S); }
+int look() { return kWaveLook; }
+int above_ids() { return kAboveIds; }
 void start() { count = IdCount{}; }
 void publish(int step, int who, int n) { count.publish(step, who, n); }
 int before(int step) { return count.before(step); }
@@ -197,3 +200,13 @@ def test_every_wait_counts_its_polls():
     assert len(waits) == 3
     for i in waits:
         assert re.search(r"give_up\(|> kWaveSpin", "\n".join(lines[i:i + 4])), lines[i]
+
+
+@pytest.mark.parametrize("S", range(1, 33))
+def test_the_row_above_has_ids_enough(ids, S):
+    """Wave 2's share of the ids covers a window's columns of the row above, all
+    distinct, with room for words that other rows keep in use."""
+    n = ids.id_count(S)
+    assert n % 128 == 0 and n <= MOST_IDS
+    own = n // 64 * (64 - ids.above_ids())
+    assert own >= 2 * S + 2 + ids.look() and own >= 24
