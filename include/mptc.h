@@ -68,7 +68,8 @@ typedef struct {
                          chains inside a tile of itile_w x 64/itile_w blocks per pass;
                          0: exhaustive search re-folds flagged blocks once per pass or, where
                          reuse chains are long (a batch with an intra frame, thresholds from
-                         5 on), decides every block once in dependency order; learned
+                         5 on, S up to 32, a sample of whose blocks reuses words widely),
+                         decides every block once in dependency order; learned
                          search uses 8 x 8 tiles (same output for every value) */
 } mptc_tuning;
 

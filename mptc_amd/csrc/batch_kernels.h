@@ -81,6 +81,7 @@ constexpr int kPassStride = 64;  // words between the group counters
 struct DevStats {
   unsigned long long inter_cands[kStatSlots * kSlot64], intra_cands[kStatSlots * kSlot64];
   unsigned long long reeval_cands[kStatSlots * kSlot64];
+  unsigned long long wave_cands[kStatSlots * kSlot64];  // k_intra_wave's positions: intra_cands unless it gave up
   unsigned long long exact_inter[kStatSlots * kSlot64], exact_intra[kStatSlots * kSlot64];  // pruned search: exact evaluations
   unsigned int n_inter[kStatSlots * kSlot32], n_intra[kStatSlots * kSlot32];
   unsigned int n_unique, active_passes;  // passes that changed a word
@@ -89,6 +90,8 @@ struct DevStats {
   unsigned int skip_tile;                // the last pass was tile-resolved (k_intra_tile_pass)
   unsigned int n_need;                   // blocks on the list of k_need_list
   unsigned int wave_ticket, wave_done, wave_fail;  // k_intra_wave: rows taken, rows finished, a row gave up
+  unsigned int wave_ok;                  // it decided every block: the kernels that take `after_wave` do nothing
+  unsigned int smp_need, smp_changed;    // k_wave_sample: blocks that search, and whose word changes
   unsigned int pass_grp[kPassGroups * kPassStride];  // pass_end's group counters
 };
 
@@ -762,9 +765,10 @@ __device__ __forceinline__ Fold fold_passing_set(const uint32_t* __restrict__ pm
 // blocks a workgroup, so that few workgroups queue on the list's counter.
 constexpr int kNeedPer = 16;
 __global__ void __launch_bounds__(256) k_need_list(const uint8_t* __restrict__ need, int total, int* __restrict__ list,
-                                                   DevStats* __restrict__ st) {
+                                                   DevStats* __restrict__ st, bool after_wave) {
   __shared__ unsigned int s_n;
   __shared__ unsigned int s_at;
+  if (after_wave && st->wave_ok) return;
   const int g0 = blockIdx.x * 256 * kNeedPer + threadIdx.x, lane = (int)(threadIdx.x & 63);
   if (threadIdx.x == 0) s_n = 0;
   __syncthreads();
@@ -801,10 +805,11 @@ __global__ void __launch_bounds__(256) k_intra_dense(const FrameDev* __restrict_
                                                      const int* __restrict__ orig, uint2* __restrict__ E4, size_t nbs,
                                                      uint4* __restrict__ summ, size_t sstride,
                                                      DevStats* __restrict__ st, const int* __restrict__ list,
-                                                     const uint8_t* __restrict__ sid) {
+                                                     const uint8_t* __restrict__ sid, bool after_wave) {
   __shared__ uint8_t s_snap[512];
   __shared__ float2 s_ab[4];
   __shared__ unsigned long long s_acc;
+  if (after_wave && st->wave_ok) return;
   int f = 0, bx = 0, by = 0, g = 0, chunk = 0;
   bool in;
   if (kList) {
@@ -876,8 +881,9 @@ __global__ void __launch_bounds__(256) k_intra_combine(const FrameDev* __restric
                                                        const uint32_t* __restrict__ cw, const uint4* __restrict__ summ,
                                                        size_t sstride, uint64_t* __restrict__ dec,
                                                        uint32_t* __restrict__ cw_new, int* __restrict__ chg_list,
-                                                       DevStats* __restrict__ st) {
+                                                       DevStats* __restrict__ st, bool after_wave) {
   __shared__ unsigned int s_base;
+  if (after_wave && st->wave_ok) return;
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   bool changed = false;
   if (g < total && need[g]) {

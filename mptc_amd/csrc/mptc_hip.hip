@@ -126,13 +126,14 @@ constexpr int kReevalGrid = 1024;  // workgroups of the re-evaluation pass (grid
 constexpr int kListGrid = 256;     // workgroups of the list-apply pass (grid-stride)
 
 struct Graphs {
-  hipGraphExec_t prefix = nullptr, passes = nullptr, wave = nullptr, suffix = nullptr;
+  hipGraphExec_t prefix = nullptr, passes = nullptr, wave = nullptr, rest = nullptr, suffix = nullptr;
   void destroy() {
     if (prefix) (void)hipGraphExecDestroy(prefix);
     if (passes) (void)hipGraphExecDestroy(passes);
     if (wave) (void)hipGraphExecDestroy(wave);
+    if (rest) (void)hipGraphExecDestroy(rest);
     if (suffix) (void)hipGraphExecDestroy(suffix);
-    prefix = passes = wave = suffix = nullptr;
+    prefix = passes = wave = rest = suffix = nullptr;
   }
 };
 // The step's graphs for a batch of intra frames only (v[0]: no inter search),
@@ -205,6 +206,7 @@ struct mptc_ctx {
   uint64_t* d_fin = nullptr;  // k_intra_wave: words, final from bit 32
   int* d_wrows = nullptr;     // its rows in ticket order (null: one frame, rows in order)
   int n_wrows = 0;
+  long wave_chain = 0;        // longest chain of its steps in a frame of the batch
   uint2* d_E = nullptr;  // S^2 groups of four int16 error deltas per block
   uint4* d_summ = nullptr;  // kMaxChunks selection summaries per block
   DevStats* d_stats = nullptr;
@@ -444,6 +446,10 @@ FrameDev frame_dev(const FrameIn& x, int tw, int ltw, int& base, int& tb, int& w
   return d;
 }
 
+// Steps of k_intra_wave over a frame: a row follows the one above by S + 2
+// blocks, or by a whole row.
+long wave_chain(int S, int bw, int bh) { return bw + (long)std::min(bw, S + 2) * bh; }
+
 // Lays out a batch (block, wave-tile and unique-tile offsets) and, when its
 // shape changed, rebuilds the block/tile frame maps and drops the graphs.
 int prepare_batch(mptc_ctx* c, hipStream_t s, int n, const FrameIn* in) {
@@ -503,7 +509,11 @@ int prepare_batch(mptc_ctx* c, hipStream_t s, int n, const FrameIn* in) {
   }
   c->n_frames = n;
   c->n_wrows = 0;
-  for (int f = 0; f < n; ++f) c->n_wrows += h[f].bh;
+  c->wave_chain = 0;
+  for (int f = 0; f < n; ++f) {
+    c->n_wrows += h[f].bh;
+    c->wave_chain = std::max(c->wave_chain, wave_chain(c->cfg.search_area, h[f].bw, h[f].bh));
+  }
   c->any_inter = false;
   c->any_intra = false;
   for (int f = 0; f < n; ++f) {
@@ -656,13 +666,41 @@ bool use_wave(const mptc_ctx* c) {
          c->cfg.err_threshold >= (S <= kWaveWideS ? kWaveMinThr : kWaveWideThr);
 }
 
+// How many of the batch's sampled blocks have to change their word at once for
+// the wave to be taken (k_wave_sample).  Frames of 64x64 to 3840x2160, S = 1 to
+// 32, thresholds 5 to 32, ms passes / wave by the share of searching blocks:
+//  - from 30 % on at S >= 8, where a changed word costs the passes 4 S^2
+//    evaluations: 640x360, S = 8, 74 % 2.15 / 1.72, 11 % 0.85 / 1.87; 1080p, S = 16,
+//    18 % 10.8 / 16.7; S = 32, 24 % 7.6 / 10.0.  20 % for short chains of steps:
+//    2048x16, S = 16, 24 % 1.63 / 0.90;
+//  - from 62 % on below: 1080p, S = 4, 59 % 2.6 / 3.1, 91 % 9.5 / 3.0, S = 2, 36 %
+//    1.1 / 2.2, 53 % 2.8 / 2.2;
+//  - from 15 % on where the wave takes about as long as ten passes: 64x64, S = 8,
+//    18 % 0.39 / 0.32, 10 % 0.17 / 0.29;
+//  - and from 8 % of all blocks on: one intra frame beside eleven inter frames,
+//    S = 8, threshold 8: 1080p, 8.5 % 25 / 14, 640x360, 1.5 % 8.0 / 13.1.
+// A sample of 1,024 blocks gives the share to 1.5 % (one standard deviation);
+// above S = 16 it is 256, to 3 %: at S = 32 a block is 4,032 evaluations.
+WaveRule wave_rule(const mptc_ctx* c) {
+  const int S = c->cfg.search_area;
+  WaveRule r;
+  r.sampled = std::min(c->total, S <= 16 ? 1024 : 256);
+  r.pct = c->wave_chain <= 200 ? 15 : S < 8 ? 62 : c->wave_chain <= 700 ? 20 : 30;
+  r.pct_all = 8;
+  return r;
+}
+
 int queue_wave(mptc_ctx* c, hipStream_t s) {
   const int S = c->cfg.search_area;
+  const WaveRule rule = wave_rule(c);
   return launch(c, s, KF_WAVE, [&] {
+    hipLaunchKernelGGL(k_wave_sample, dim3(rule.sampled), dim3(256), 0, s, c->d_fr, c->d_sid, c->total,
+                       rule.sampled, S, c->cfg.err_threshold, c->d_own, c->d_need, c->d_cw, c->d_ctab, c->d_orig,
+                       c->d_stats);
     auto kern = S == 8 ? k_intra_wave<8> : S == 16 ? k_intra_wave<16> : S == 32 ? k_intra_wave<32> : k_intra_wave<0>;
     hipLaunchKernelGGL(kern, dim3(c->n_wrows), dim3(64 * kWaveWaves), wave_dims(S).bytes, s, c->d_fr,
                        c->n_frames > 1 ? c->d_wrows : nullptr, S, c->cfg.err_threshold, c->d_summ, c->d_ctab,
-                       c->d_fin, c->d_intra, c->d_stats, c->d_conv);
+                       c->d_fin, c->d_intra, c->d_stats, c->d_conv, rule);
   });
 }
 
@@ -680,9 +718,13 @@ int queue_intra_prep(mptc_ctx* c, hipStream_t s, bool prune, bool wave, const ui
   });
 }
 
-// The three launch sequences of a step.  `fit` = false starts from
-// caller-provided fitted blocks already in d_own; `wave`: k_intra_wave follows
-// (no intra candidates evaluated here).
+int queue_intra_search(mptc_ctx* c, hipStream_t s, bool x_done, bool after_wave);
+
+// The launch sequences of a step.  `fit` = false starts from caller-provided
+// fitted blocks already in d_own; `wave`: k_intra_wave follows (no intra
+// candidates evaluated here), and queue_intra_search after it, whose kernels do
+// nothing if the wave decided the batch: queued beside it, they follow without
+// a gap if it did not.
 int queue_prefix(mptc_ctx* c, hipStream_t s, bool fit, bool wave) {
   const int total = c->total, wg = c->tune.wg_size, tw = c->tune.tile_w;
   const int S = c->cfg.search_area, thr = c->cfg.err_threshold;
@@ -747,7 +789,17 @@ int queue_prefix(mptc_ctx* c, hipStream_t s, bool fit, bool wave) {
       return rc;
   }
   if (!prep_done && (rc = queue_intra_prep(c, s, prune, wave, inter_summ, orig_ready))) return rc;
-  if (wave) return MPTC_OK;
+  return wave ? MPTC_OK : queue_intra_search(c, s, x_done, false);
+}
+
+// The intra candidates against the starting words, and the first decisions.
+int queue_intra_search(mptc_ctx* c, hipStream_t s, bool x_done, bool after_wave) {
+  const int total = c->total, wg = c->tune.wg_size, tw = c->tune.tile_w;
+  const int S = c->cfg.search_area, thr = c->cfg.err_threshold, K = window_chunks(c);
+  const unsigned gwk = grid_for(c->n_wtiles * K * 64, wg);
+  const unsigned gwk256 = grid_for(c->n_wtiles * K * 64, 256);
+  const bool prune = use_prune(c);
+  int rc;
   if (c->mode == MPTC_SEARCH_LEARNED) {
     if ((rc = proposals_q(c, s, MPTC_NET_INTRA, c->d_need, c->d_prop, x_done))) return rc;
     return lintra_pass_q(c, s, 0, 1, false);
@@ -784,17 +836,17 @@ int queue_prefix(mptc_ctx* c, hipStream_t s, bool fit, bool wave) {
   if ((rc = launch(c, s, KF_DENSE, [&] {
          if (listed)
            hipLaunchKernelGGL(k_need_list, dim3(grid_for(total, 256 * kNeedPer)), dim3(256), 0, s, c->d_need, total,
-                              c->d_chg, c->d_stats);
+                              c->d_chg, c->d_stats, after_wave);
          auto kern = listed ? k_intra_dense<true> : k_intra_dense<false>;
          hipLaunchKernelGGL(kern, dim3(listed ? grid_for((total + 63) / 64 * K * 64, wg) : gwk), dim3(wg), 0, s,
                             c->d_fr, c->d_tsid, c->n_wtiles, tw, K, S, c->d_own, c->d_need, c->d_cw, c->d_ctab,
-                            c->d_orig, c->d_E, c->nbs, c->d_summ, c->nbs, c->d_stats, c->d_chg, c->d_sid);
+                            c->d_orig, c->d_E, c->nbs, c->d_summ, c->nbs, c->d_stats, c->d_chg, c->d_sid, after_wave);
        })))
     return rc;
   if ((rc = launch(c, s, KF_INTRA_COMBINE, [&] {
          hipLaunchKernelGGL(k_intra_combine, dim3(grid_for(total, wg)), dim3(wg), 0, s, c->d_fr, c->d_sid, total, K,
                             S, thr, c->d_own, c->d_need, c->d_cw, c->d_summ, c->nbs, c->d_intra, c->d_cwn, c->d_chg,
-                            c->d_stats);
+                            c->d_stats, after_wave);
        })))
     return rc;
   return launch(c, s, KF_APPLY, [&] {
@@ -897,7 +949,9 @@ int run_step(mptc_ctx* c, hipStream_t s, bool fit) {
   if (graphs && !gr.prefix) {
     if ((rc = capture(s, &gr.prefix, [&] { return queue_prefix(c, s, true, wave); }))) return rc;
     if ((rc = capture(s, &gr.passes, [&] { return queue_passes(c, s); }))) return rc;
-    if (wave && (rc = capture(s, &gr.wave, [&] { return queue_wave(c, s); }))) return rc;
+    if (wave && ((rc = capture(s, &gr.wave, [&] { return queue_wave(c, s); })) ||
+                 (rc = capture(s, &gr.rest, [&] { return queue_intra_search(c, s, false, true); }))))
+      return rc;
     if ((rc = capture(s, &gr.suffix, [&] { return queue_suffix(c, s); }))) return rc;
   }
   if (graphs) {
@@ -917,8 +971,8 @@ int run_step(mptc_ctx* c, hipStream_t s, bool fit) {
     if (q != hipSuccess) return fail(MPTC_EHIP, std::string("hipEventQuery: ") + hipGetErrorString(q));
     return MPTC_OK;
   };
-  // k_intra_wave over the whole batch; false in `ok`: a window held more
-  // distinct words than it has ids for, and the passes start over
+  // k_intra_wave over the whole batch; false in `ok`: few blocks reuse words, or
+  // a window held more distinct ones than it has ids for, and the passes follow
   auto run_wave = [&](bool& ok) -> int {
     int r;
     if (graphs) {
@@ -927,9 +981,14 @@ int run_step(mptc_ctx* c, hipStream_t s, bool fit) {
       return r;
     }
     HIP_TRY(hipEventRecord(c->batch_ev[0], s));
+    if (graphs) {
+      HIP_TRY(hipGraphLaunch(gr.rest, s));
+    } else if ((r = queue_intra_search(c, s, false, true))) {
+      return r;
+    }
     if ((r = wait(0))) return r;
     ok = *conv == 0;
-    return ok ? MPTC_OK : queue_prefix(c, s, fit, false);
+    return MPTC_OK;
   };
   bool settled = false;
   if (wave && (rc = run_wave(settled))) return rc;
@@ -1274,7 +1333,7 @@ int32_t mptc_get_stats(mptc_ctx* c, mptc_frame_stats* out) {
     out->n_inter += d.n_inter[i * kSlot32];
     out->n_intra += d.n_intra[i * kSlot32];
     out->inter_candidates += (int64_t)d.inter_cands[i * kSlot64];
-    out->intra_candidates += (int64_t)d.intra_cands[i * kSlot64];
+    out->intra_candidates += (int64_t)d.intra_cands[i * kSlot64] + (d.wave_fail ? 0 : (int64_t)d.wave_cands[i * kSlot64]);
     out->reeval_candidates += (int64_t)d.reeval_cands[i * kSlot64];
     out->exact_inter_candidates += (int64_t)d.exact_inter[i * kSlot64];
     out->exact_intra_candidates += (int64_t)d.exact_intra[i * kSlot64];
@@ -1853,6 +1912,7 @@ int32_t mptc_encode_frame_noalloc(int32_t device, const uint8_t* d_rgb, int32_t 
   c->any_intra = is_intra;
   c->last_intra = is_intra;
   c->n_wrows = nd.h_fr.bh;
+  c->wave_chain = wave_chain(search_area, nd.h_fr.bw, nd.h_fr.bh);
   // the status word of the passes or the wave comes back by a plain copy (no
   // event, no mapped memory)
   auto status = [&]() -> int {
@@ -1868,9 +1928,8 @@ int32_t mptc_encode_frame_noalloc(int32_t device, const uint8_t* d_rgb, int32_t 
   for (int passes = 0; !settled;) {
     if (wave) {
       wave = false;
-      if ((rc = queue_wave(c, s)) || (rc = status())) return rc;
+      if ((rc = queue_wave(c, s)) || (rc = queue_intra_search(c, s, false, true)) || (rc = status())) return rc;
       settled = nd.h_changed == 0;
-      if (!settled && (rc = queue_prefix(c, s, true, false))) return rc;
       continue;
     }
     if (passes > c->total + 4 * np) return fail(MPTC_ESTATE, "intra fixpoint did not converge");

@@ -138,3 +138,74 @@ def test_small_windows_have_ids_enough(enc, orc, S, thr):
     rgb = _frame("soft", 480, 256, 40 + S)
     _intra(enc, orc, rgb, S, thr)
     assert enc.stats()["intra_iterations"] == 1
+
+
+def _route(enc, run):
+    """The call's result and whether the fixpoint passes followed the wave."""
+    enc.profile_enable(True)
+    got = run()
+    passes = enc.profile_read("intra_reeval")[0]
+    enc.profile_enable(False)
+    return got, passes > 0
+
+
+# content and size by which a batch is left to the passes: hardly any reuse, and words that change for few blocks
+@pytest.mark.parametrize("kind,w,h,S,thr,passes", [
+    ("noise", 320, 200, 8, 8, True), ("noise", 64, 64, 16, 8, True), ("noise", 320, 200, 4, 32, True),
+    ("noise", 200, 200, 32, 8, True), ("flat", 400, 300, 16, 5, True), ("soft", 400, 300, 8, 8, False),
+    ("soft", 64, 64, 8, 32, False), ("soft", 300, 200, 32, 16, False), ("soft", 400, 300, 5, 32, False)])
+def test_route_by_reuse(enc, orc, kind, w, h, S, thr, passes):
+    log(f"{kind} {w}x{h} S={S} thr={thr}")
+    _, by_passes = _route(enc, lambda: _intra(enc, orc, _frame(kind, w, h, w + S), S, thr))
+    assert by_passes == passes
+
+
+def _window(bw, bh, S):
+    """Intra window positions of a frame whose blocks all search."""
+    return sum(min(y, 2 * S - 1) * (min(bw, x + S) - max(0, x - S)) + x - max(0, x - S) for y in range(bh) for x in range(bw))
+
+
+# edges of the window, its rings, staging groups and polled vectors, with words that most blocks reuse
+@pytest.mark.parametrize("w,h,S", [(68, 400, 1), (200, 200, 1), (260, 160, 3), (16, 240, 8), (60, 40, 8), (252, 64, 8), (256, 64, 8),
+                                   (260, 64, 7), (200, 100, 9), (220, 96, 15), (220, 96, 16), (260, 132, 17), (300, 140, 31),
+                                   (300, 140, 32)])
+def test_edges_with_wide_reuse(enc, orc, w, h, S):
+    log(f"{w}x{h} S={S}")
+    _, by_passes = _route(enc, lambda: _intra(enc, orc, _frame("soft", w, h, w + h), S, 64))
+    assert not by_passes
+    assert enc.stats()["intra_candidates"] == _window(w // 4, h // 4, S)
+
+
+def test_ids_run_out_in_a_frame_of_wide_reuse(enc, orc):
+    """Reuse over half a frame and noise in the other: the wave begins, a window
+    holds more distinct words than ids, and the passes take the frame."""
+    w, h, S = 400, 300, 32
+    rgb = _frame("soft", w, h, 6)
+    rgb[:, w // 2:] = _frame("noise", w, h, 7)[:, w // 2:]
+    _, by_passes = _route(enc, lambda: _intra(enc, orc, rgb, S, 8))
+    assert by_passes
+    assert enc.stats()["intra_candidates"] == _window(w // 4, h // 4, S)
+
+
+def test_small_intra_frame_among_inter_frames(enc, orc):
+    """An intra frame of few blocks does not send the batch's inter frames
+    through the wave."""
+    from mptc_amd import hip
+    S, thr = 8, 8
+    enc.set_params(S, thr)
+    jobs, want = [], []
+    for i, (w, h, intra) in enumerate([(32, 32, True), (400, 300, False), (400, 300, False)]):
+        a = _frame("soft", w, h, 10 + i)
+        b = np.clip(a.astype(int) + _frame("noise", w, h, 20 + i) % 5 - 2, 0, 255).astype(np.uint8)
+        nb = (w // 4) * (h // 4)
+        ref = orc.reencode(a, orc.fit_frame(a), S, thr, True)["phys"]
+        want.append(orc.reencode(b, orc.fit_frame(b), S, thr, intra, None if intra else ref))
+        jobs.append(dict(d_rgb=hip.Buffer.from_array(b), width=w, height=h, is_intra=intra, d_ref=hip.Buffer.from_array(ref),
+                         d_phys=hip.Buffer(8 * nb), d_motion=hip.Buffer(2 * nb), d_unique=hip.Buffer(4 * nb),
+                         d_n_unique=hip.Buffer(4), d_eps=hip.Buffer(6 * nb), d_kind=hip.Buffer(nb)))
+    _, by_passes = _route(enc, lambda: enc.encode_batch_device(jobs))
+    assert by_passes
+    for i, (j, wnt) in enumerate(zip(jobs, want)):
+        nb = (j["width"] // 4) * (j["height"] // 4)
+        assert np.array_equal(j["d_phys"].download(np.uint64, nb), wnt["phys"]), f"frame {i}"
+        assert np.array_equal(j["d_motion"].download(np.uint8, 2 * nb), wnt["motion"]), f"frame {i}"
