@@ -60,9 +60,10 @@ typedef struct {
                          this many runs scanned by separate waves, 1..8 (4 or
                          more is taken as 8 in small batches, and above threshold
                          4 the inter search of S = 8..16 takes 8) */
-  int32_t prune;      /* 1: for thresholds 0..4 (batches of intra frames alone: 0..2,
-                         above S = 16 0..1), evaluate exactly only the candidates an
-                         error lower bound cannot rule out (same output);
+  int32_t prune;      /* 1: for thresholds 0..4 (the intra search of a batch of which
+                         intra frames hold a quarter or more: above S = 8 0..2, above
+                         S = 16 0..1), evaluate exactly only the candidates an error
+                         lower bound cannot rule out (same output);
                          0: evaluate every candidate */
   int32_t itile_w;    /* intra fixpoint passes: 8, 16, 32 or 64: a wave settles the reuse
                          chains inside a tile of itile_w x 64/itile_w blocks per pass;

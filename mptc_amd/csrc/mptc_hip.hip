@@ -137,9 +137,10 @@ struct Graphs {
   }
 };
 // The step's graphs for a batch of intra frames only (v[0]: no inter search),
-// of inter frames only (v[1]) and of both (v[2]).
+// of inter frames only (v[1]) and of both, its intra search pruned (v[2]) or
+// not (v[3]).
 struct GraphSet {
-  Graphs v[3];
+  Graphs v[4];
   void destroy() {
     for (Graphs& g : v) g.destroy();
   }
@@ -226,6 +227,7 @@ struct mptc_ctx {
   GraphSet graphs;
   bool any_inter = true;   // the batch holds an inter frame
   bool any_intra = false;  // and an intra frame
+  int intra_blocks = 0;    // blocks in its intra frames
   int last_passes = 0, last_total = 0, last_intra = 0;
   // learned proposals
   int mode = MPTC_SEARCH_EXHAUSTIVE, top_k = 8;
@@ -516,7 +518,9 @@ int prepare_batch(mptc_ctx* c, hipStream_t s, int n, const FrameIn* in) {
   }
   c->any_inter = false;
   c->any_intra = false;
+  c->intra_blocks = 0;
   for (int f = 0; f < n; ++f) {
+    if (in[f].is_intra) c->intra_blocks += h[f].nb;
     c->any_inter = c->any_inter || !in[f].is_intra;
     c->any_intra = c->any_intra || in[f].is_intra;
   }
@@ -535,20 +539,28 @@ int prepare_batch(mptc_ctx* c, hipStream_t s, int n, const FrameIn* in) {
 // streams, threshold 8: 5.5 ms so, 4.4 with every candidate evaluated.
 constexpr int kPruneMaxThr = 4;
 
-//
-// In a batch of intra frames alone the fixpoint passes, which keep the passing
-// sets up to date, grow with the threshold while the bound's share shrinks; the
-// search is pruned up to threshold 2, above S = 16 up to 1.  Intra frames, ms
-// pruned / not: 1080p S = 8 threshold 0 0.48 / 0.60, 2 1.16 / 1.20, 3 2.11 / 2.11;
-// 768x700 S = 16 0 0.94 / 1.05, 2 2.62 / 2.53, 3 4.92 / 4.17, 4 8.4 / 6.8, S = 8
-// 4 2.2 / 2.0; 1204x668 S = 32 2 23.4 / 20.1, 4 77 / 54.
-int prune_max_thr(const mptc_ctx* c) {
-  return c->any_inter ? kPruneMaxThr : c->cfg.search_area <= 16 ? 2 : 1;
+// Whether the context's settings let a batch's searches be pruned.
+bool prune_set(const mptc_ctx* c) {
+  return c->tune.prune && c->mode == MPTC_SEARCH_EXHAUSTIVE && !c->record && c->cfg.err_threshold >= 0 &&
+         c->cfg.err_threshold <= kPruneMaxThr;
 }
 
-bool use_prune(const mptc_ctx* c) {
-  return c->tune.prune && c->mode == MPTC_SEARCH_EXHAUSTIVE && !c->record && c->cfg.err_threshold >= 0 &&
-         c->cfg.err_threshold <= prune_max_thr(c) && c->total <= 1 << 27;  // 32-bit offsets of the words' tables
+// The batch's inter search.
+bool prune_inter(const mptc_ctx* c) {
+  return prune_set(c) && c->any_inter && c->total <= 1 << 27;  // 32-bit offsets of the words' tables
+}
+
+// Its intra search.  Where intra frames hold a quarter of the blocks or more, the
+// fixpoint passes, which keep the passing sets up to date, grow with the threshold
+// and the window while the bound's share shrinks: it is pruned up to threshold 2
+// above S = 8 and up to 1 above 16 (an inter frame's few searching blocks: up to
+// 4).  Intra frames, ms pruned / not: 640x360, gradients with noise, S = 8
+// threshold 4 1.42 / 1.32; S = 16 2 2.4 / 2.8, 4 6.0 / 5.3; S = 32 1 5.0 / 7.5, 4
+// 21.1 / 18.8; and noise, which reuses nothing, S = 8 4 0.10 / 0.14, 1280x720 0.12 /
+// 0.25.
+bool prune_intra(const mptc_ctx* c) {
+  const int S = c->cfg.search_area, most = S <= 8 ? kPruneMaxThr : S <= 16 ? 2 : 1;
+  return prune_set(c) && c->total <= 1 << 27 && (c->cfg.err_threshold <= most || 4LL * c->intra_blocks < c->total);
 }
 
 // The inter search by distinct words (k_inter_words): plain searches above the
@@ -735,13 +747,14 @@ int queue_prefix(mptc_ctx* c, hipStream_t s, bool fit, bool wave) {
                        (c->mode == MPTC_SEARCH_LEARNED && !c->net[MPTC_NET_INTRA].use_prior));
   bool x_done = want_x;
   bool prep_done = false;  // need and the starting intra words already set
-  const bool prune = use_prune(c);  // (no wave then: its thresholds are higher)
+  // (no wave then: its thresholds are higher)
+  const bool prune_p = prune_inter(c), prune_i = prune_intra(c);
   if ((rc = launch(c, s, KF_FIT, [&] {
          const int n_st = (int)(sizeof(DevStats) / 4);
          hipLaunchKernelGGL(k_block_prep, dim3(grid_for(std::max(total, n_st + c->n_tiles), wg)), dim3(wg), 0, s,
                             c->d_fr, c->d_sid, total, fit ? c->d_own : nullptr, c->d_rw, c->d_rtab,
                             want_x ? c->ew.X : nullptr, reinterpret_cast<uint32_t*>(c->d_stats), n_st, c->d_tiles,
-                            c->n_tiles, prune ? c->d_rbt : nullptr);
+                            c->n_tiles, prune_p ? c->d_rbt : nullptr);
        })))
     return rc;
   const int K = window_chunks(c);
@@ -753,7 +766,7 @@ int queue_prefix(mptc_ctx* c, hipStream_t s, bool fit, bool wave) {
   const unsigned gwk256 = grid_for(c->n_wtiles * K * 64, 256);
   if (!c->any_inter) {
     // a batch of intra frames only: no inter search (k_intra_prep reads no inter decision)
-  } else if (prune) {
+  } else if (prune_p) {
     // inter: bound (tables from k_block_prep), exact evaluation of the
     // survivors, fold (prune_kernels.h)
     if ((rc = launch(c, s, KF_PRUNED_INTER, [&] {
@@ -788,7 +801,7 @@ int queue_prefix(mptc_ctx* c, hipStream_t s, bool fit, bool wave) {
          })))
       return rc;
   }
-  if (!prep_done && (rc = queue_intra_prep(c, s, prune, wave, inter_summ, orig_ready))) return rc;
+  if (!prep_done && (rc = queue_intra_prep(c, s, prune_i, wave, inter_summ, orig_ready))) return rc;
   return wave ? MPTC_OK : queue_intra_search(c, s, x_done, false);
 }
 
@@ -798,13 +811,12 @@ int queue_intra_search(mptc_ctx* c, hipStream_t s, bool x_done, bool after_wave)
   const int S = c->cfg.search_area, thr = c->cfg.err_threshold, K = window_chunks(c);
   const unsigned gwk = grid_for(c->n_wtiles * K * 64, wg);
   const unsigned gwk256 = grid_for(c->n_wtiles * K * 64, 256);
-  const bool prune = use_prune(c);
   int rc;
   if (c->mode == MPTC_SEARCH_LEARNED) {
     if ((rc = proposals_q(c, s, MPTC_NET_INTRA, c->d_need, c->d_prop, x_done))) return rc;
     return lintra_pass_q(c, s, 0, 1, false);
   }
-  if (prune) {  // bound tables and (up to S = 8) cleared passing sets from k_intra_prep
+  if (prune_intra(c)) {  // bound tables and (up to S = 8) cleared passing sets from k_intra_prep
     if (S > 8 && (rc = launch(c, s, KF_PREP, [&] {
           hipLaunchKernelGGL(k_zero16, dim3(2048), dim3(256), 0, s, reinterpret_cast<uint4*>(c->d_pm),
                              (size_t)total * pass_words(S) / 4);
@@ -830,9 +842,9 @@ int queue_intra_search(mptc_ctx* c, hipStream_t s, bool x_done, bool after_wave)
                          c->d_stats);
     });
   }
-  // a batch with inter frames above the pruned thresholds: a lane per searching
-  // block (listed in d_chg, which the combine fills afterwards)
-  const bool listed = c->any_inter && thr > kPruneMaxThr;
+  // a batch with inter frames, not pruned: a lane per searching block (listed in
+  // d_chg, which the combine fills afterwards)
+  const bool listed = c->any_inter && (prune_inter(c) || thr > kPruneMaxThr);
   if ((rc = launch(c, s, KF_DENSE, [&] {
          if (listed)
            hipLaunchKernelGGL(k_need_list, dim3(grid_for(total, 256 * kNeedPer)), dim3(256), 0, s, c->d_need, total,
@@ -870,7 +882,7 @@ int queue_passes(mptc_ctx* c, hipStream_t s) {
     return MPTC_OK;
   }
   // the pruned search keeps passing sets beside E (prune_kernels.h)
-  uint32_t* pm = use_prune(c) ? c->d_pm : nullptr;
+  uint32_t* pm = prune_intra(c) ? c->d_pm : nullptr;
   // itile_w 0: re-fold passes (no skip in k_intra_reeval; skip_tile stays 0)
   const int tw_log = itile_log(c);
   for (int p = 0; p < np; ++p) {
@@ -937,7 +949,7 @@ int capture(hipStream_t s, hipGraphExec_t* exec, Q&& q) {
 // One encode step over the prepared batch.
 int run_step(mptc_ctx* c, hipStream_t s, bool fit) {
   const bool graphs = c->tune.use_graph && !c->prof && fit;
-  Graphs& gr = c->graphs.v[!c->any_inter ? 0 : c->any_intra ? 2 : 1];
+  Graphs& gr = c->graphs.v[!c->any_inter ? 0 : !c->any_intra ? 1 : prune_intra(c) ? 2 : 3];
   int rc;
   // The last pass of each batch writes its count of changed words to h_conv
   // (0 when it had nothing to do).  Passes of an earlier step that are still
@@ -1037,7 +1049,7 @@ int encode_batch(mptc_ctx* c, hipStream_t s, int n, const FrameIn* in, bool fit)
   int rc = join_stream(c, s);
   if (rc) return rc;
   if ((rc = prepare_batch(c, s, n, in))) return rc;
-  if (use_prune(c) && (rc = prune_ensure(c))) return rc;
+  if ((prune_inter(c) || prune_intra(c)) && (rc = prune_ensure(c))) return rc;
   c->last_intra = n == 1 ? in[0].is_intra : 0;
   if ((rc = run_step(c, s, fit))) return rc;
   return leave_stream(c, s);
@@ -1267,7 +1279,7 @@ int32_t mptc_autotune(mptc_ctx* c, int32_t n, const mptc_frame_io* frames, int32
   mptc_tuning probe = keep;
   probe.prune = 1;
   c->tune = probe;
-  const int n_prune = use_prune(c) ? 2 : 1;
+  const int n_prune = prune_inter(c) || prune_intra(c) ? 2 : 1;
   // times the shape t (warm-up: maps and graphs; then `steps` encodes) and keeps the fastest
   auto trial = [&](const mptc_tuning& t) -> int {
     c->tune = t;
@@ -1910,6 +1922,7 @@ int32_t mptc_encode_frame_noalloc(int32_t device, const uint8_t* d_rgb, int32_t 
   c->n_itiles = lt;
   c->any_inter = !is_intra;
   c->any_intra = is_intra;
+  c->intra_blocks = is_intra ? nd.h_fr.nb : 0;
   c->last_intra = is_intra;
   c->n_wrows = nd.h_fr.bh;
   c->wave_chain = wave_chain(search_area, nd.h_fr.bw, nd.h_fr.bh);

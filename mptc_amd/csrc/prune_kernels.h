@@ -273,7 +273,7 @@ __global__ void __launch_bounds__(256) k_pruned_search(const FrameDev* __restric
         const int i = kIntra ? bx + S - 1 - t - u : bx - S + t + u;
         const int ic = min(max(i, 0), fbw - 1);  // clamped into the frame: the load is always in bounds
         there[u] = row_in & (i == ic) & !(kIntra && r == 0 && t + u < S);
-        // 32-bit offset into the frame's tables (use_prune: batches of at most 2^27 blocks)
+        // 32-bit offset into the frame's tables (batches of at most 2^27 blocks)
         tb4[u] = *reinterpret_cast<const BoundTab*>(ftab + (uint32_t)(row_at + ic) * (uint32_t)sizeof(BoundTab));
       }
 #pragma unroll

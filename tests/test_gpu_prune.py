@@ -70,3 +70,43 @@ def test_bounded_positions_are_the_window_inside_the_frame(enc, orc, w, h, S):
     enc.set_tuning()
     assert counts[0] == counts[1]
     assert counts[1][0] in (window, 2 * window)  # of the last frame, or of both where the counts run on
+
+
+def _batch(lib, hip, orc, e, frames, flags, S, thr):
+    """One call with frames[1:], intra or inter by flag, each inter frame after frames[0]; checked against the oracle."""
+    h, w = frames.shape[1:3]
+    nb = (w // 4) * (h // 4)
+    ref = orc.reencode(frames[0], orc.fit_frame(frames[0]), S, thr, True)["phys"]
+    jobs = [dict(d_rgb=hip.Buffer.from_array(np.ascontiguousarray(f)), width=w, height=h, is_intra=flag,
+                 d_ref=hip.Buffer.from_array(ref), d_phys=hip.Buffer(8 * nb), d_motion=hip.Buffer(2 * nb),
+                 d_unique=hip.Buffer(4 * nb), d_n_unique=hip.Buffer(4), d_eps=hip.Buffer(6 * nb), d_kind=hip.Buffer(nb))
+            for f, flag in zip(frames[1:], flags)]
+    e.encode_batch_device(jobs)
+    for i, (j, f, flag) in enumerate(zip(jobs, frames[1:], flags)):
+        want = orc.reencode(f, orc.fit_frame(f), S, thr, flag, None if flag else ref)
+        assert np.array_equal(j["d_phys"].download(np.uint64, nb), want["phys"]), (flags, i)
+        assert np.array_equal(j["d_motion"].download(np.uint8, 2 * nb), want["motion"]), (flags, i)
+    return e.stats()
+
+
+# whether the intra search of a batch of these frames is pruned: small windows, thresholds up to the limit, few intra blocks
+@pytest.mark.parametrize("S,thr,flags,pruned", [
+    (8, 4, "IIIII", True), (8, 3, "IPPPP", True), (16, 2, "IIPPP", True), (16, 3, "IPPPP", True), (16, 3, "IIPPP", False),
+    (16, 4, "IIIII", False), (16, 4, "PPPPP", True), (24, 1, "IIIPP", True), (24, 2, "IIIPP", False), (24, 4, "IPPPP", True)])
+@pytest.mark.parametrize("graph", [0, 1])
+def test_intra_search_pruned_by_its_share(orc, S, thr, flags, pruned, graph):
+    """The inter search is pruned wherever there is one, the intra search by its
+    limit; with graphs, calls of one shape and other flags follow each other."""
+    from mptc_amd import hip, lib
+    w, h = 100, 60
+    frames = orc.synth_frames(SynthCfg(w, h, S + thr, 5, 1, 3, 8, 0), 6)
+    e = lib.Encoder(w, h, search_area=S, err_threshold=thr, max_batch_frames=5, max_batch_blocks=5 * (w // 4) * (h // 4))
+    e.set_tuning(use_graph=graph)
+    for _ in range(2):
+        st = _batch(lib, hip, orc, e, frames, [c == "I" for c in flags], S, thr)
+        assert (st["exact_inter_candidates"] > 0) == ("P" in flags)
+        assert (st["exact_intra_candidates"] > 0) == pruned
+        if graph:
+            _batch(lib, hip, orc, e, frames, [c == "I" for c in "IIIPI"], S, thr)
+            _batch(lib, hip, orc, e, frames, [c == "I" for c in "PIPPP"], S, thr)
+    e.close()
