@@ -1275,11 +1275,12 @@ int32_t mptc_autotune(mptc_ctx* c, int32_t n, const mptc_frame_io* frames, int32
   const int wgs[] = {64, 128, 256};
   const int tws[] = {64, 32, 16, 8};
   const int chunks[] = {1, 2, 4, 8};
-  // the pruned search is tried where it applies (both give the same output)
+  // the pruned searches are tried where the settings let them apply (both give the same output); whether they do to
+  // these frames shows when they are encoded
   mptc_tuning probe = keep;
   probe.prune = 1;
   c->tune = probe;
-  const int n_prune = prune_inter(c) || prune_intra(c) ? 2 : 1;
+  const int n_prune = prune_set(c) ? 2 : 1;
   // times the shape t (warm-up: maps and graphs; then `steps` encodes) and keeps the fastest
   auto trial = [&](const mptc_tuning& t) -> int {
     c->tune = t;

@@ -110,3 +110,23 @@ def test_intra_search_pruned_by_its_share(orc, S, thr, flags, pruned, graph):
             _batch(lib, hip, orc, e, frames, [c == "I" for c in "IIIPI"], S, thr)
             _batch(lib, hip, orc, e, frames, [c == "I" for c in "PIPPP"], S, thr)
     e.close()
+
+
+def test_autotune_tries_pruning_whatever_ran_before(orc):
+    """A context last used for intra frames that are not pruned finds the pruned
+    inter search, which is about twice as fast here."""
+    from mptc_amd import hip, lib
+    S, thr, w, h = 16, 3, 640, 360
+    nb = (w // 4) * (h // 4)
+    frames = orc.synth_frames(SynthCfg(w, h, 3, 5, 1, 3, 8, 0), 2)
+    e = lib.Encoder(w, h, search_area=S, err_threshold=thr)
+    ref = hip.Buffer(8 * nb)
+    out = [hip.Buffer(2 * nb), hip.Buffer(4 * nb), hip.Buffer(4), hip.Buffer(6 * nb), hip.Buffer(nb)]
+    e.encode_frame_device(hip.Buffer.from_array(frames[0]), w, h, True, None, ref, *out)
+    assert e.stats()["exact_intra_candidates"] == 0
+    e.set_tuning(prune=0)
+    job = dict(d_rgb=hip.Buffer.from_array(frames[1]), width=w, height=h, is_intra=False, d_ref=ref, d_phys=hip.Buffer(8 * nb),
+               d_motion=out[0], d_unique=out[1], d_n_unique=out[2], d_eps=out[3], d_kind=out[4])
+    best, _ = e.autotune([job], 1)
+    assert best["prune"] == 1
+    e.close()
