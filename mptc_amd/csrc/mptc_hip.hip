@@ -205,7 +205,7 @@ struct mptc_ctx {
   float4 *d_rtab = nullptr, *d_ctab = nullptr;
   int *d_orig = nullptr, *d_chg = nullptr;
   uint64_t* d_fin = nullptr;  // k_intra_wave: words, final from bit 32
-  int* d_wrows = nullptr;     // its rows in ticket order (null: one frame, rows in order)
+  int* d_wrows = nullptr;     // its rows in ticket order (batches of several frames)
   int n_wrows = 0;
   long wave_chain = 0;        // longest chain of its steps in a frame of the batch
   uint2* d_E = nullptr;  // S^2 groups of four int16 error deltas per block
@@ -476,36 +476,29 @@ int prepare_batch(mptc_ctx* c, hipStream_t s, int n, const FrameIn* in) {
   HIP_TRY(hipMemcpyAsync(c->d_fr, h, sizeof(FrameDev) * n, hipMemcpyHostToDevice, s));
   const bool same = shape == c->shape && std::memcmp(&c->tune, &c->shape_tune, sizeof(mptc_tuning)) == 0;
   if (!same) {
+    c->shape.clear();  // a failure below leaves no shape that a later call could match
+    c->graphs.destroy();
     // frame index of every wave tile
     std::vector<uint8_t> tsid(std::max(wt, 1));
     for (int f = 0; f < n; ++f) {
       const int cnt = h[f].tiles_x * ((h[f].bh + (64 / tw) - 1) / (64 / tw));
       std::fill(tsid.begin() + h[f].wtile_base, tsid.begin() + h[f].wtile_base + cnt, (uint8_t)f);
     }
-    if (c->d_tsid) (void)hipFree(c->d_tsid);
-    c->d_tsid = nullptr;
-    int rc = dalloc(&c->d_tsid, tsid.size());
-    if (rc) return rc;
     HIP_TRY(hipMemcpyAsync(c->d_tsid, tsid.data(), tsid.size(), hipMemcpyHostToDevice, s));
     int maxnb = 1;
     for (int f = 0; f < n; ++f) maxnb = std::max(maxnb, h[f].nb);
     hipLaunchKernelGGL(k_fill_sid, dim3(grid_for(maxnb, 256), n), dim3(256), 0, s, c->d_fr, n, c->d_sid);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(s));  // the tsid staging vector is released on return
-    if (c->d_wrows) (void)hipFree(c->d_wrows);
-    c->d_wrows = nullptr;
+    std::vector<int> rows;
     if (n > 1) {  // k_intra_wave's rows: every frame's first, then every frame's second, ...
-      std::vector<int> rows;
       int maxh = 0;
       for (int f = 0; f < n; ++f) maxh = std::max(maxh, h[f].bh);
       for (int y = 0; y < maxh; ++y)
         for (int f = 0; f < n; ++f)
           if (y < h[f].bh) rows.push_back(y << 6 | f);
-      if ((rc = dalloc(&c->d_wrows, rows.size()))) return rc;
       HIP_TRY(hipMemcpyAsync(c->d_wrows, rows.data(), sizeof(int) * rows.size(), hipMemcpyHostToDevice, s));
-      HIP_TRY(hipStreamSynchronize(s));
     }
-    c->graphs.destroy();
+    HIP_TRY(hipStreamSynchronize(s));  // the staging vectors are released on return
     c->shape = shape;
     c->shape_tune = c->tune;
   }
@@ -1114,6 +1107,8 @@ int32_t mptc_create(const mptc_config* cfg, mptc_ctx** out) {
       (rc = dalloc(&c->d_rw, nb)) || (rc = dalloc(&c->d_cw, nb)) || (rc = dalloc(&c->d_cwn, nb)) ||
       (rc = dalloc(&c->d_dirty, nb)) || (rc = dalloc(&c->d_tiles, max_tiles)) || (rc = dalloc(&c->d_rtab, nb)) ||
       (rc = dalloc(&c->d_ctab, nb)) || (rc = dalloc(&c->d_orig, nb)) || (rc = dalloc(&c->d_chg, nb)) || (rc = dalloc(&c->d_fin, nb)) ||
+      // a wave tile and a block row hold a block at least
+      (rc = dalloc(&c->d_tsid, nb)) || (rc = dalloc(&c->d_wrows, nb)) ||
       (rc = dalloc(&c->d_E, groups * c->nbs)) || (rc = dalloc(&c->d_summ, kMaxChunks * c->nbs)) || (rc = dalloc(&c->d_stats, 1)) ||
       (rc = dalloc(&c->d_rgb, one_nb * 48)) || (rc = dalloc(&c->d_ref, one_nb)) || (rc = dalloc(&c->d_phys, one_nb)) ||
       (rc = dalloc(&c->d_motion, one_nb * 2)) || (rc = dalloc(&c->d_eps, one_nb * 6)) ||

@@ -231,3 +231,32 @@ def test_learned_batch_matches_single_streams(orc):
             assert np.array_equal(res[f][i]["kind"], one[f][0]["kind"])
             reused += int((res[f][i]["kind"] != 0).sum())
     assert reused > 0
+
+
+def test_batches_of_changing_shapes(orc):
+    """Calls of one context whose frame counts and sizes change, with a refused
+    call between: every batch is laid out anew."""
+    from mptc_amd import hip, lib
+    S, thr = 8, 8
+    e = lib.Encoder(128, 128, search_area=S, err_threshold=thr, max_batch_frames=4, max_batch_blocks=4 * 32 * 32)
+
+    def job(w, h, seed):
+        yy, xx = np.mgrid[0:h, 0:w]
+        r = np.random.default_rng(seed)
+        f = np.clip(np.stack([30 + xx, 60 + yy, 200 - xx // 2], -1) + r.integers(-8, 9, (h, w, 3)), 0, 255).astype(np.uint8)
+        nb = (w // 4) * (h // 4)
+        return f, dict(d_rgb=hip.Buffer.from_array(f), width=w, height=h, is_intra=True, d_ref=None, d_phys=hip.Buffer(8 * nb),
+                       d_motion=hip.Buffer(2 * nb), d_unique=hip.Buffer(4 * nb), d_n_unique=hip.Buffer(4),
+                       d_eps=hip.Buffer(6 * nb), d_kind=hip.Buffer(nb))
+
+    sizes = [[(128, 128)], [(64, 32), (128, 100), (4, 4)], [(128, 100), (64, 32), (4, 4)], [(32, 128)] * 4, [(64, 32), (128, 100), (4, 4)]]
+    for k, dims in enumerate(sizes):
+        made = [job(w, h, 10 * k + i) for i, (w, h) in enumerate(dims)]
+        bad = dict(made[-1][1], width=made[-1][1]["width"] + 2)
+        with pytest.raises(Exception):
+            e.encode_batch_device([j for _, j in made[:-1]] + [bad])
+        e.encode_batch_device([j for _, j in made])
+        for i, (f, j) in enumerate(made):
+            want = orc.reencode(f, orc.fit_frame(f), S, thr, True)
+            assert np.array_equal(j["d_phys"].download(np.uint64, len(want["phys"])), want["phys"]), (k, i)
+    e.close()
