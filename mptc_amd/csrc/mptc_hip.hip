@@ -238,7 +238,8 @@ struct mptc_ctx {
   uint4* d_h2p = nullptr;     // layer-2 activations of the step (net_infer.h tiles)
   int16_t* d_pinter = nullptr;  // inter proposals, kMaxTopK per block
   int16_t* d_prop = nullptr;    // intra proposals, kMaxTopK per block
-  // pruned exhaustive search (prune_kernels.h), allocated on first use
+  // pruned exhaustive search (prune_kernels.h), allocated on first use if there is room
+  bool prune_room = true;
   BoundTab *d_rbt = nullptr, *d_cbt = nullptr;  // bound tables of reference / current words
   uint32_t* d_pm = nullptr;                      // passing sets of the intra windows (pass_words(alloc_S) per block)
   bool record = false;          // exhaustive steps record acceptance masks
@@ -534,8 +535,8 @@ constexpr int kPruneMaxThr = 4;
 
 // Whether the context's settings let a batch's searches be pruned.
 bool prune_set(const mptc_ctx* c) {
-  return c->tune.prune && c->mode == MPTC_SEARCH_EXHAUSTIVE && !c->record && c->cfg.err_threshold >= 0 &&
-         c->cfg.err_threshold <= kPruneMaxThr;
+  return c->tune.prune && c->prune_room && c->mode == MPTC_SEARCH_EXHAUSTIVE && !c->record &&
+         c->cfg.err_threshold >= 0 && c->cfg.err_threshold <= kPruneMaxThr;
 }
 
 // The batch's inter search.
@@ -586,14 +587,21 @@ int window_chunks(const mptc_ctx* c) {
 // Chunk summaries the exhaustive inter search leaves per block.
 int inter_chunks(const mptc_ctx* c) { return use_words(c) ? kWordsWaves : window_chunks(c); }
 
-int prune_ensure(mptc_ctx* c) {
-  if (c->d_rbt) return MPTC_OK;
+// The pruned searches' tables, on first use: 64 bytes a block and the passing
+// sets (32 bytes at S = 8, 2 KB at 63).  Without room for them the context's
+// searches stay unpruned (same output).
+void prune_ensure(mptc_ctx* c) {
+  if (c->d_rbt) return;
   const size_t nb = (size_t)c->max_total;
-  int rc;
-  if ((rc = dalloc(&c->d_rbt, nb)) || (rc = dalloc(&c->d_cbt, nb)) ||
-      (rc = dalloc(&c->d_pm, nb * pass_words(c->alloc_S))))
-    return rc;
-  return MPTC_OK;
+  if (dalloc(&c->d_rbt, nb) == MPTC_OK && dalloc(&c->d_cbt, nb) == MPTC_OK &&
+      dalloc(&c->d_pm, nb * pass_words(c->alloc_S)) == MPTC_OK)
+    return;
+  (void)hipGetLastError();  // the allocation's error is dealt with
+  if (c->d_rbt) (void)hipFree(c->d_rbt);
+  if (c->d_cbt) (void)hipFree(c->d_cbt);
+  c->d_rbt = c->d_cbt = nullptr;
+  c->d_pm = nullptr;
+  c->prune_room = false;
 }
 
 // Inference over X -> H2 tiles (d_h2p) -> the top-kk admitted offsets of each
@@ -1042,7 +1050,7 @@ int encode_batch(mptc_ctx* c, hipStream_t s, int n, const FrameIn* in, bool fit)
   int rc = join_stream(c, s);
   if (rc) return rc;
   if ((rc = prepare_batch(c, s, n, in))) return rc;
-  if ((prune_inter(c) || prune_intra(c)) && (rc = prune_ensure(c))) return rc;
+  if (prune_inter(c) || prune_intra(c)) prune_ensure(c);
   c->last_intra = n == 1 ? in[0].is_intra : 0;
   if ((rc = run_step(c, s, fit))) return rc;
   return leave_stream(c, s);

@@ -130,3 +130,25 @@ def test_autotune_tries_pruning_whatever_ran_before(orc):
     best, _ = e.autotune([job], 1)
     assert best["prune"] == 1
     e.close()
+
+
+def test_context_without_room_for_the_pruned_tables(orc):
+    """A context that takes most of the free memory, with no room for the pruned
+    searches' tables, encodes as before, with every candidate evaluated."""
+    import ctypes as C
+
+    from mptc_amd import hip, lib
+    S, w, h = 63, 64, 64
+    free, total = C.c_size_t(), C.c_size_t()
+    hip.check(hip.rt().hipMemGetInfo(C.byref(free), C.byref(total)))
+    # a block of the context: E, 8 chunk summaries, words, tables and maps; the pruned tables are 6 % more
+    per_block = 8 * S * S + 8 * 16 + 116
+    blocks = int(0.955 * free.value) // per_block
+    assert blocks * (64 + 1984) > free.value - blocks * per_block + (1 << 28)
+    e = lib.Encoder(w, h, search_area=S, err_threshold=0, max_batch_frames=1, max_batch_blocks=blocks)
+    frames = orc.synth_frames(SynthCfg(w, h, 3, 5, 1, 3, 8, 0), 2)
+    for _ in range(2):
+        for x, y in zip(e.encode_sequence(frames, 8), orc.encode_sequence(frames, S, 0, 8)):
+            compare_results(x, y, "no room")
+        assert e.stats()["exact_inter_candidates"] == 0
+    e.close()
