@@ -1,7 +1,7 @@
 """Benchmark: MPTC per-frame encode throughput (Mblocks/s) at 1080p on one MI355X,
 plain (bit-exact) search vs learned-proposal search, with the PSNR delta.
 
-python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu-baseline] [--no-learned]
+python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu-baseline] [--no-learned] [--record FILE]
 
 Workload: the 1080p sequence (64 frames of 1920x1080 RGB8 from the seeded
 generator: gradient, 32 rectangles with velocities in [-4, 4] px/frame, 1 %
@@ -17,7 +17,9 @@ offsets pass its accept test on 1080p training sequences of other seeds (and
 how often an offset passes by the number of pixel indices its word differs
 from the block's own), both proposal networks are trained on the GPU, and the
 same K steps are encoded with top-4 proposals (the inter ranking adding the
-index-similarity scores; exact acceptance).  Prints one JSON line.
+index-similarity scores; exact acceptance).  Prints one JSON line of the
+results, short enough for a log's tail; --record FILE writes the whole record
+(kernels, work, training, frontiers, the configs' rooflines) as well.
 """
 from __future__ import annotations
 
@@ -74,6 +76,7 @@ def parse():
     ap.add_argument("--no-threshold8", action="store_true", help="skip the learned frontier at threshold 8")
     ap.add_argument("--train-steps", type=int, default=3000)
     ap.add_argument("--workload", default=WORKLOAD)
+    ap.add_argument("--record", help="write the whole record to this file (the printed line is its short form)")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="only run a device-to-device copy of known size (rocprof counter scale)")
     return ap.parse_args()
@@ -803,6 +806,26 @@ def measure_learned(hip, lib, enc, R, spec, a, value, work, psnr_plain, tuning):
     return learned
 
 
+def short_line(out: dict) -> dict:
+    """The printed part of the record `out`: the workload, its figures and one
+    figure of each further measurement."""
+    keys = ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling",
+            "vs_baseline", "dtype", "data", "config", "psnr_db", "bit_exact", "bit_exact_frames_checked")
+    s = {k: out[k] for k in keys}
+    s["config"] = {k: out["config"][k] for k in ("workload", "blocks_per_frame")}
+    s["roofline"] = {k: out["roofline"][k] for k in ("kernel", "bound", "achieved", "peak", "unit", "frac")}
+    s["end_to_end"] = [out[k]["value"] for k in ("end_to_end", "end_to_end_overlapped")]
+    if "learned" in out:
+        s["learned"] = {k: out["learned"][k] for k in ("top_k", "value", "speedup_vs_plain", "reuse_recall", "psnr_delta_db")}
+    if "config3" in out:
+        s["config3_ms"] = {k: v["ms_per_step"] for k, v in out["config3"]["results"].items()}
+    if "config4" in out:
+        s["config4_ms"] = out["config4"]["ms_per_step"]
+    if "gpu_over_cpu" in out:
+        s["gpu_over_cpu"] = out["gpu_over_cpu"]
+    return s
+
+
 def main():
     a = parse()
     if a.gpus != 1:
@@ -933,7 +956,10 @@ def main():
         out["gpu_over_cpu"] = round(value / allc["value"], 1)
         out["gpu_over_cpu_1core"] = round(value / one["value"], 1)
     note("done")
-    print(json.dumps(out), flush=True)
+    if a.record:
+        with open(a.record, "w") as fh:
+            json.dump(out, fh)
+    print(json.dumps(short_line(out)), flush=True)
     enc.close()
 
 
