@@ -431,7 +431,7 @@ constexpr uint32_t kNoWord = 0xFFFFu;
 // 2 S / 8 window rows of every block through the rule, with the deltas
 // looked up.  The evaluations bound it: at S = 8, threshold 8, a tile's 511
 // positions hold 128 words where a block has 256 candidates (S = 16: 297 of
-// 1,446, and 1,024).  Twelve streams, 1.5 million blocks, S = 8, threshold 8:
+// 1,446, and 1,024).  Twelve streams, 2.16 million blocks, S = 8, threshold 8:
 // 4.2 ms by candidate, 2.4 so.  Requesting the pixels ahead of the window's
 // words takes registers from the evaluations (3.0 ms).
 // A tile with more than WordsDims::ids words evaluates candidate by candidate.

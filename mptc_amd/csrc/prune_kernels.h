@@ -55,7 +55,6 @@
 
 namespace mptc {
 
-
 // Pixel side of the bound for one block.
 struct BoundBlk {
   uint32_t pc[12];  // pc[3j + ch]: channel ch of pixels 4j..4j+3, less 128, signed bytes

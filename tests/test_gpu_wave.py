@@ -209,3 +209,20 @@ def test_small_intra_frame_among_inter_frames(enc, orc):
         nb = (j["width"] // 4) * (j["height"] // 4)
         assert np.array_equal(j["d_phys"].download(np.uint64, nb), wnt["phys"]), f"frame {i}"
         assert np.array_equal(j["d_motion"].download(np.uint8, 2 * nb), wnt["motion"]), f"frame {i}"
+
+
+@pytest.mark.parametrize("kind,S,thr", [("soft", 8, 8), ("soft", 3, 32), ("noise", 8, 8), ("flat", 5, 6)])
+def test_allocation_free_call_takes_the_same_routes(orc, kind, S, thr):
+    from mptc_amd import hip, lib
+    w, h = 300, 200
+    nb = (w // 4) * (h // 4)
+    rgb = _frame(kind, w, h, 30 + S)
+    d_rgb = hip.Buffer.from_array(rgb)
+    o = [hip.Buffer(8 * nb), hip.Buffer(2 * nb), hip.Buffer(4 * nb), hip.Buffer(4), hip.Buffer(6 * nb), hip.Buffer(nb)]
+    stream = hip.Stream()
+    want = orc.reencode(rgb, orc.fit_frame(rgb), S, thr, True)
+    for _ in range(2):
+        lib.encode_frame_noalloc(0, d_rgb, w, h, S, thr, True, None, *o, stream=stream.handle)
+        assert np.array_equal(o[0].download(np.uint64, nb), want["phys"])
+        assert np.array_equal(o[1].download(np.uint8, 2 * nb), want["motion"])
+    stream.destroy()
