@@ -68,6 +68,7 @@ struct FrameDev {
 constexpr int kStatSlots = 32;
 constexpr int kSlot64 = 16;
 constexpr int kSlot32 = 32;
+constexpr int kSmpSlots = 16;
 
 // pass_end counts finished workgroups in two levels: at most kPassGroups groups
 // of at least kPassGroup workgroups count into their own counter (one 256-byte
@@ -91,7 +92,7 @@ struct DevStats {
   unsigned int n_need;                   // blocks on the list of k_need_list
   unsigned int wave_ticket, wave_done, wave_fail;  // k_intra_wave: rows taken, rows finished, a row gave up
   unsigned int wave_ok;                  // it decided every block: the kernels that take `after_wave` do nothing
-  unsigned int smp_need, smp_changed;    // k_wave_sample: blocks that search, and whose word changes
+  unsigned int smp[kSmpSlots * kSlot32];  // k_wave_sample: blocks that search, and << 16 those whose word changes
   unsigned int pass_grp[kPassGroups * kPassStride];  // pass_end's group counters
 };
 

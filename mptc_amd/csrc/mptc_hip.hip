@@ -707,7 +707,7 @@ int queue_wave(mptc_ctx* c, hipStream_t s) {
   const int S = c->cfg.search_area;
   const WaveRule rule = wave_rule(c);
   return launch(c, s, KF_WAVE, [&] {
-    hipLaunchKernelGGL(k_wave_sample, dim3(rule.sampled), dim3(256), 0, s, c->d_fr, c->d_sid, c->total,
+    hipLaunchKernelGGL(k_wave_sample, dim3(rule.sampled), dim3(S <= 8 ? 256 : S <= 16 ? 512 : 1024), 0, s, c->d_fr, c->d_sid, c->total,
                        rule.sampled, S, c->cfg.err_threshold, c->d_own, c->d_need, c->d_cw, c->d_ctab, c->d_orig,
                        c->d_stats);
     auto kern = S == 8 ? k_intra_wave<8> : S == 16 ? k_intra_wave<16> : S == 32 ? k_intra_wave<32> : k_intra_wave<0>;

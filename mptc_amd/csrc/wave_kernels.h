@@ -243,13 +243,14 @@ __device__ __forceinline__ T gload(const T* p) {
 
 // Whether the blocks of a batch reuse words widely enough for k_intra_wave: n
 // blocks spread over it take their first decision (from the starting words, as
-// k_intra_dense), a workgroup each; smp_need counts those that search,
-// smp_changed those whose word changes.  Where few change the fixpoint passes
+// k_intra_dense), a workgroup each; smp counts those that search and those whose
+// word changes, in 16 slots (one word for all workgroups: 28 us at 1,024 blocks).  Where few change the fixpoint passes
 // settle after a handful of rounds, while the wave's time is its chain of steps
 // whatever the frame holds (1080p, S = 8, threshold 8: noise, 0 % changed, passes
 // 0.41 ms, wave 5.6; 24 grey levels, 11 %, 1.9 and 5.7; gradients with noise,
-// 96 %, 21.5 and 4.7).
-__global__ void __launch_bounds__(256) k_wave_sample(const FrameDev* __restrict__ fr, const uint8_t* __restrict__ sid,
+// 96 %, 21.5 and 4.7).  A thread takes up to four positions (S = 32: 16 of them,
+// one after the other, 37 us; four, 28; S = 8, one, 9.7 us).
+__global__ void __launch_bounds__(1024) k_wave_sample(const FrameDev* __restrict__ fr, const uint8_t* __restrict__ sid,
                                                      int total, int n, int S, int thr,
                                                      const uint64_t* __restrict__ own, const uint8_t* __restrict__ need,
                                                      const uint32_t* __restrict__ cw, const float4* __restrict__ ctab,
@@ -311,10 +312,12 @@ __global__ void __launch_bounds__(256) k_wave_sample(const FrameDev* __restrict_
     sel = m != kNone && (m >> 12) - 32768 <= thr ? m & 4095 : kNone;
   }
   if (lane != 0) return;
-  atomicAdd(&st->smp_need, 1u);
-  if (sel == kNone) return;
-  const int r = sel / W2, x = bx + S - 1 - (sel - r * W2);
-  if (cw[d.base + (by - r) * bw + x] != cw[g]) atomicAdd(&st->smp_changed, 1u);
+  bool changed = false;
+  if (sel != kNone) {
+    const int r = sel / W2, x = bx + S - 1 - (sel - r * W2);
+    changed = cw[d.base + (by - r) * bw + x] != cw[g];
+  }
+  atomicAdd(&st->smp[i % kSmpSlots * kSlot32], changed ? 0x10001u : 1u);
 }
 
 // Least share of blocks that change, of those of the sample that search (the
@@ -339,8 +342,11 @@ __global__ void __launch_bounds__(64 * kWaveWaves) k_intra_wave(
     const float4* __restrict__ ctab, uint64_t* fin, uint64_t* __restrict__ dec, DevStats* __restrict__ st,
     unsigned int* __restrict__ conv, WaveRule rule) {
   {  // not worth it (k_wave_sample): the passes take the batch
-    const int changed = (int)st->smp_changed;
-    if (changed * 100 < rule.pct * (int)st->smp_need || changed * 100 < rule.pct_all * rule.sampled) {
+    uint32_t smp = 0;
+#pragma unroll
+    for (int i = 0; i < kSmpSlots; ++i) smp += st->smp[i * kSlot32];
+    const int changed = (int)(smp >> 16), need = (int)(smp & 0xFFFFu);
+    if (changed * 100 < rule.pct * need || changed * 100 < rule.pct_all * rule.sampled) {
       if (blockIdx.x == 0 && threadIdx.x == 0 && conv) {
         *reinterpret_cast<volatile unsigned int*>(conv) = 1u;
         __threadfence_system();
