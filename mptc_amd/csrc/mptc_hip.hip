@@ -806,8 +806,6 @@ int queue_prefix(mptc_ctx* c, hipStream_t s, bool fit, bool wave) {
   return wave ? MPTC_OK : queue_intra_search(c, s, x_done, false);
 }
 
-constexpr int kListMinS = 5;
-
 // The intra candidates against the starting words, and the first decisions.
 int queue_intra_search(mptc_ctx* c, hipStream_t s, bool x_done, bool after_wave) {
   const int total = c->total, wg = c->tune.wg_size, tw = c->tune.tile_w;
@@ -846,10 +844,12 @@ int queue_intra_search(mptc_ctx* c, hipStream_t s, bool x_done, bool after_wave)
     });
   }
   // a batch with inter frames, not pruned: a lane per searching block (listed in
-  // d_chg, which the combine fills afterwards).  Below S = 5 a block's candidates
-  // are fewer than the list costs: 1080p inter, threshold 8, us without / with it,
-  // noise S = 2 170 / 181, S = 4 269 / 275; gradients with noise, S = 16, 2,897 / 2,663.
-  const bool listed = c->any_inter && S >= kListMinS && (prune_inter(c) || thr > kPruneMaxThr);
+  // d_chg, which the combine fills afterwards).  Few candidates in all, at S up to
+  // 4, cost less than the launch that makes the list: 1080p inter, threshold 8, us
+  // without / with it, noise S = 2 170 / 181, S = 4 269 / 275; gradients with noise,
+  // S = 4, twelve such frames 2,414 / 1,886; S = 16 2,897 / 2,663.
+  const bool few = S <= 4 && 4LL * S * S * total < 1 << 24;
+  const bool listed = c->any_inter && !few && (prune_inter(c) || thr > kPruneMaxThr);
   if ((rc = launch(c, s, KF_DENSE, [&] {
          if (listed)
            hipLaunchKernelGGL(k_need_list, dim3(grid_for(total, 256 * kNeedPer)), dim3(256), 0, s, c->d_need, total,
