@@ -226,3 +226,28 @@ def test_allocation_free_call_takes_the_same_routes(orc, kind, S, thr):
         assert np.array_equal(o[0].download(np.uint64, nb), want["phys"])
         assert np.array_equal(o[1].download(np.uint8, 2 * nb), want["motion"])
     stream.destroy()
+
+
+def test_replayed_graphs_take_the_route_of_each_frame(orc):
+    """Graphs captured on one frame are replayed on others of its shape: frames
+    for the wave, for the passes, and one that the wave gives up on, in turn."""
+    from mptc_amd import hip, lib
+    S, thr, w, h = 32, 8, 320, 240
+    nb = (w // 4) * (h // 4)
+    mixed = _frame("soft", w, h, 6)
+    mixed[:, w // 2:] = _frame("noise", w, h, 7)[:, w // 2:]
+    frames = [_frame("soft", w, h, 5), _frame("noise", w, h, 8), mixed, _frame("soft", w, h, 9)]
+    want = [orc.reencode(f, orc.fit_frame(f), S, thr, True) for f in frames]
+    e = lib.Encoder(w, h, S, thr)
+    e.set_tuning(use_graph=1)
+    d = [hip.Buffer.from_array(f) for f in frames]
+    o = [hip.Buffer(8 * nb), hip.Buffer(2 * nb), hip.Buffer(4 * nb), hip.Buffer(4), hip.Buffer(6 * nb), hip.Buffer(nb)]
+    its = []
+    for k in (0, 1, 2, 3, 1, 0, 2, 0):
+        e.encode_frame_device(d[k], w, h, True, None, *o)
+        e.synchronize()
+        assert np.array_equal(o[0].download(np.uint64, nb), want[k]["phys"]), k
+        assert np.array_equal(o[1].download(np.uint8, 2 * nb), want[k]["motion"]), k
+        its.append((k, e.stats()["intra_iterations"]))
+    assert all((n == 1) == (k in (0, 3)) for k, n in its), its
+    e.close()
